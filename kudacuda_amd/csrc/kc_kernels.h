@@ -178,6 +178,13 @@ struct Nf4GemmArgs {
     float eps = 1e-6f;
 };
 hipError_t launch_nf4_gemm(GemmEpi epi, const Nf4GemmArgs& args, hipStream_t stream);
+// The second half of a split GEMM: a.partials [weights][splits][m][n] summed in
+// split order, then the epilogue.
+hipError_t launch_nf4_gemm_reduce(GemmEpi epi, const Nf4GemmArgs& args, int64_t splits, hipStream_t stream);
+// The same product for any token count (kc_gemm.hip), for calls that
+// nf4_tile_gemm_fits() accepts.
+bool nf4_tile_gemm_fits(GemmEpi epi, const Nf4GemmArgs& args);
+hipError_t launch_nf4_tile_gemm(GemmEpi epi, const Nf4GemmArgs& args, hipStream_t stream);
 
 // Row RMSNorm of m rows of 2048: out[r] = bf16((x[r] * inv_rms) * gamma), the
 // decode kernels' fp32 order.  With `embed`, row r is embed[tokens[start + r]]

@@ -546,6 +546,23 @@ __global__ __launch_bounds__(256) void residual_norm_reduce_kernel(Nf4GemmArgs a
     *reinterpret_cast<uint4*>(a.norm_out + m * a.n + c) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
 }
 
+// The split partials of one GEMM summed in split order, with its epilogue.
+template <GemmEpi EPI>
+hipError_t launch_reduce(const Nf4GemmArgs& a, int64_t S, hipStream_t stream) {
+    const int64_t quads = a.m * a.n / 4;
+    if constexpr (EPI == GemmEpi::kQkvRope) {
+        hipLaunchKernelGGL(qkv_rope_reduce_kernel, dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0,
+                           stream, a, static_cast<int>(S));
+    } else if constexpr (EPI == GemmEpi::kResidualNorm) {
+        hipLaunchKernelGGL(residual_norm_reduce_kernel, dim3(static_cast<unsigned>(a.m)), dim3(256), 0, stream, a,
+                           static_cast<int>(S));
+    } else {
+        hipLaunchKernelGGL(gemm_reduce_kernel<EPI>, dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0,
+                           stream, a, static_cast<int>(S));
+    }
+    return hipGetLastError();
+}
+
 template <GemmEpi EPI>
 hipError_t launch_gemm_epi(const Nf4GemmArgs& a, hipStream_t stream) {
     constexpr int NF = EPI == GemmEpi::kSwiGlu ? 2 : 1;
@@ -611,18 +628,7 @@ hipError_t launch_gemm_epi(const Nf4GemmArgs& a, hipStream_t stream) {
     if (status != hipSuccess || S == 1) {
         return status;
     }
-    const int64_t quads = a.m * a.n / 4;
-    if constexpr (EPI == GemmEpi::kQkvRope) {
-        hipLaunchKernelGGL(qkv_rope_reduce_kernel, dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0,
-                           stream, a, static_cast<int>(S));
-    } else if constexpr (EPI == GemmEpi::kResidualNorm) {
-        hipLaunchKernelGGL(residual_norm_reduce_kernel, dim3(static_cast<unsigned>(a.m)), dim3(256), 0, stream, a,
-                           static_cast<int>(S));
-    } else {
-        hipLaunchKernelGGL(gemm_reduce_kernel<EPI>, dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0,
-                           stream, a, static_cast<int>(S));
-    }
-    return hipGetLastError();
+    return launch_reduce<EPI>(a, S, stream);
 }
 
 }  // namespace
@@ -662,6 +668,22 @@ hipError_t launch_nf4_gemm(GemmEpi epi, const Nf4GemmArgs& a, hipStream_t stream
             return launch_gemm_epi<GemmEpi::kQkvRope>(a, stream);
         case GemmEpi::kResidualNorm:
             return launch_gemm_epi<GemmEpi::kResidualNorm>(a, stream);
+    }
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_nf4_gemm_reduce(GemmEpi epi, const Nf4GemmArgs& a, int64_t splits, hipStream_t stream) {
+    switch (epi) {
+        case GemmEpi::kBias:
+            return launch_reduce<GemmEpi::kBias>(a, splits, stream);
+        case GemmEpi::kResidual:
+            return launch_reduce<GemmEpi::kResidual>(a, splits, stream);
+        case GemmEpi::kSwiGlu:
+            return launch_reduce<GemmEpi::kSwiGlu>(a, splits, stream);
+        case GemmEpi::kQkvRope:
+            return launch_reduce<GemmEpi::kQkvRope>(a, splits, stream);
+        case GemmEpi::kResidualNorm:
+            return launch_reduce<GemmEpi::kResidualNorm>(a, splits, stream);
     }
     return hipErrorInvalidValue;
 }

@@ -1,0 +1,112 @@
+"""GPU: the NF4 GEMM for more than 64 tokens (csrc/kc_gemm.hip).
+
+Sizes pick every block shape of its dispatch and the edges of each: a last
+token tile with one token, a last row tile half empty, one K window, an odd
+number of windows, split and unsplit K.  The reference sums the same
+bf16-rounded weights in fp64; the bound is one bf16 step of the output
+(tests/test_gpu_prefill.py::_close).
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from tests._gpu_util import dev, empty, host, p
+from tests.test_gpu_prefill import _acts, _bf16_ulps_apart, _close, _weights
+
+pytestmark = pytest.mark.gpu
+SEED = 20260901
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (65, 64, 128),       # low blocks: one window a K-group, half a row tile, one token in the last tile
+    (129, 192, 2048),    # low, split K
+    (300, 320, 384),     # low by the short k, three windows
+    (300, 192, 4224),    # square blocks, split K
+    (257, 2112, 4224),   # square, unsplit row tiles past half the chip
+    (705, 6208, 128),    # wide blocks: two windows, a quarter of the last row tile
+    (1025, 4160, 384),   # wide, one token in the last tile
+])
+@pytest.mark.parametrize("epi", ["plain", "bias", "residual"])
+def test_nf4_gemm_of_many_tokens_matches_fp64(torch_gpu, native, stream, m, n, k, epi):
+    torch = torch_gpu
+    rng = np.random.default_rng([SEED, m, n, k])
+    print(f"nf4_gemm m={m} n={n} k={k} epi={epi}", flush=True)
+    packed, absmax, wbf = _weights(rng, n, k)
+    xb, x = _acts(rng, m, k)
+    acc = (x @ wbf.T).astype(np.float32)
+    bias = O.f32_to_bf16((rng.standard_normal(n) * 0.02).astype(np.float32))
+    res = O.f32_to_bf16(rng.standard_normal((m, n)).astype(np.float32))
+    want = {"plain": acc, "bias": acc + O.bf16_to_f32(bias),
+            "residual": O.bf16_to_f32(res) + O.bf16_to_f32(O.f32_to_bf16(acc))}[epi]
+    d_x, d_w, d_a, d_b = (dev(torch, t) for t in (xb, packed, absmax, bias))
+    out = dev(torch, res) if epi == "residual" else empty(torch, m * n, "u16")  # residual in place
+    native.call("kudacuda_nf4_gemm_bf16", p(d_x), p(d_w), p(d_a), p(d_b) if epi == "bias" else 0,
+                p(out) if epi == "residual" else 0, p(out), m, k, n, 64, stream.cuda_stream)
+    stream.synchronize()
+    _close(host(out).reshape(m, n), want, inner=acc if epi == "residual" else None)
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (65, 64, 256),       # pair blocks, split K, half a row tile
+    (127, 192, 128),     # pair, one window a K-group
+    (1100, 1984, 128),   # wide blocks, half the last row tile
+    (1025, 1920, 384),   # wide, six windows, one token in the last tile
+])
+def test_nf4_gemm_swiglu_of_many_tokens_matches_fp64(torch_gpu, native, stream, m, n, k):
+    torch = torch_gpu
+    rng = np.random.default_rng([SEED, 7, m, n, k])
+    print(f"nf4_gemm_swiglu m={m} n={n} k={k}", flush=True)
+    gp, ga, gw = _weights(rng, n, k, std=0.06)
+    up, ua, uw = _weights(rng, n, k, std=0.06)
+    xb, x = _acts(rng, m, k)
+    want = O.silu((x @ gw.T).astype(np.float32)) * (x @ uw.T).astype(np.float32)
+    out = empty(torch, m * n, "u16")
+    bufs = [dev(torch, t) for t in (xb, gp, ga, up, ua)]
+    native.call("kudacuda_nf4_gemm_swiglu_bf16", *[p(b) for b in bufs], p(out), m, k, n, 64, stream.cuda_stream)
+    stream.synchronize()
+    _close(host(out).reshape(m, n), want)
+
+
+@pytest.mark.parametrize("count", [200, 301, 900, 1700])
+def test_prefill_rows_equal_those_of_64_token_parts(torch_gpu, native, count):
+    """One layer: a long prompt at once (q, k, v in low, square, pair and wide
+    blocks) writes the cache rows that its 64-token parts write, to the bound
+    of test_gpu_prefill (0.2 % of the elements more than one bf16 step apart)."""
+
+    from kudacuda_amd import synthetic
+    from kudacuda_amd.qwen2_decoder import Qwen2Nf4Decoder
+
+    torch = torch_gpu
+    gpu = Qwen2Nf4Decoder.synthetic(native, torch, seed=SEED, num_layers=1, vocab=512, kv_capacity=1728,
+                                    token_capacity=1728)
+    try:
+        lib = native.lib
+        prompt = synthetic.prompt_ids(SEED, count, 512)
+        print(f"prefill of {count} tokens in 64-token parts and at once", flush=True)
+        nbytes = int(lib.kudacuda_qwen2_prefill_workspace_bytes(64))
+        ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda:0")
+        gpu.reset(prompt)
+        for start in range(0, count, 64):
+            part = min(64, count - start)
+            native.check(lib.kudacuda_qwen2_model_prefill(gpu.model, ws.data_ptr(), nbytes, start, part,
+                                                          gpu.stream.cuda_stream), "prefill")
+        gpu.stream.synchronize()
+        names = ("key_cache", "value_cache")
+        parts = [O.bf16_to_f32(host(gpu.layers[0][n]).reshape(2, -1, 128)[:, :count]) for n in names]
+        logits = O.bf16_to_f32(host(gpu.logits))
+        for n in names:
+            gpu.layers[0][n].zero_()
+        torch.cuda.synchronize()
+        gpu.prefill(prompt)
+        gpu.stream.synchronize()
+        for n, want in zip(names, parts):
+            got = O.bf16_to_f32(host(gpu.layers[0][n]).reshape(2, -1, 128)[:, :count])
+            far = int(np.count_nonzero(_bf16_ulps_apart(got, want) > 1))
+            print(f"{n}: {far} of {got.size} more than one bf16 step apart", flush=True)
+            assert far <= 0.002 * got.size
+        assert float(np.abs(O.bf16_to_f32(host(gpu.logits)) - logits).max()) <= 0.03
+    finally:
+        gpu.close()
