@@ -215,8 +215,16 @@ struct PrefillAttnArgs {
     int64_t start = 0;
     int64_t m = 0;
     float qk_scale_log2 = 0.0f;
+    float* partials = nullptr;  // scratch of the matrix-core kernel's key splits
+    int64_t partial_floats = 0;
 };
+// One block per query row and half of its heads: up to kAttnRowKeys cached rows.
+constexpr int64_t kAttnRowKeys = 128;
 hipError_t launch_prefill_attention(const PrefillAttnArgs& args, hipStream_t stream);
+// The same on the matrix cores (kc_prefill_attn.hip), for calls that
+// prefill_attention_mfma_fits() accepts.
+bool prefill_attention_mfma_fits(const PrefillAttnArgs& args);
+hipError_t launch_prefill_attention_mfma(const PrefillAttnArgs& args, hipStream_t stream);
 // control[0] = step, stop state cleared (control[4], control[5] = 0); capture-safe
 hipError_t launch_set_step(int32_t* control, int32_t step, hipStream_t stream);
 
