@@ -185,6 +185,9 @@ hipError_t launch_nf4_gemm_reduce(GemmEpi epi, const Nf4GemmArgs& args, int64_t 
 // nf4_tile_gemm_fits() accepts.
 bool nf4_tile_gemm_fits(GemmEpi epi, const Nf4GemmArgs& args);
 hipError_t launch_nf4_tile_gemm(GemmEpi epi, const Nf4GemmArgs& args, hipStream_t stream);
+// The same for few tokens (kc_gemm_few.hip), for calls that nf4_few_gemm_fits() accepts.
+bool nf4_few_gemm_fits(GemmEpi epi, const Nf4GemmArgs& args);
+hipError_t launch_nf4_few_gemm(GemmEpi epi, const Nf4GemmArgs& args, hipStream_t stream);
 
 // Row RMSNorm of m rows of 2048: out[r] = bf16((x[r] * inv_rms) * gamma), the
 // decode kernels' fp32 order.  With `embed`, row r is embed[tokens[start + r]]

@@ -638,17 +638,18 @@ bool gemm_shape_ok(Handle* h, const char* symbol, int64_t tokens, int64_t in_fea
     return true;
 }
 
-// More than kGemmMaxTokens tokens go through the tile kernel, which forms each
-// weight once per 64 or 128 tokens in one launch; fewer (and calls it cannot
-// take: unaligned buffers) in launches of kGemmMaxTokens rows, whose waves
-// keep a 16-row fragment for all of them (gate/up of 64 tokens there 23.3 us, of
-// 65 in the tile kernel 25.3; of 65 in two of those launches 39).
+// Few tokens (up to 64, more where they still make one round of its blocks) go
+// through kc_gemm_few.hip, more through the tile kernel, which forms each weight
+// once per 64 or 128 tokens in one launch.  Calls that neither can take (unaligned
+// buffers; k no multiple of 256 at up to 64 tokens) go in launches of
+// kGemmMaxTokens rows, whose waves keep a 16-row fragment for all of them.
 hipError_t gemm_chunks(GemmEpi epi, Nf4GemmArgs a, int64_t tokens, hipStream_t stream) {
-    if (tokens > kGemmMaxTokens) {
-        a.m = tokens;
-        if (nf4_tile_gemm_fits(epi, a)) {
-            return launch_nf4_tile_gemm(epi, a, stream);
-        }
+    a.m = tokens;
+    if (nf4_few_gemm_fits(epi, a)) {
+        return launch_nf4_few_gemm(epi, a, stream);
+    }
+    if (tokens > kGemmMaxTokens && nf4_tile_gemm_fits(epi, a)) {
+        return launch_nf4_tile_gemm(epi, a, stream);
     }
     const uint16_t* x = a.x;
     const uint16_t* res = a.residual;
