@@ -488,6 +488,223 @@ void gqa_partial_kernel_f16(const uint16_t* k_rows, const uint16_t* v_rows, cons
     gqa_partial_body<F16>(k_rows, v_rows, q_vec, kv_len_device, capacity, args);
 }
 
+// The round path for the decode step's long form (gqa_merge_kernel merges), where
+// a split has several rounds: the same operations in the same order for every
+// head, with the rounds of a span side by side instead of one after the other.
+// Grid (max_splits, 2, 4): block (s, g, z) owns query heads 2z and 2z + 1 of KV
+// head g over split s, in spans of up to 8 rounds: all rows requested at once, all
+// scores, then every round's weights against its running maximum (a prefix of the
+// rounds' maxima), then the weighted sums in token order, a thread per (head, dim).
+// Three barriers a span instead of two a round.
+// What bounds it: two dependent memory trips (kv_len, rows) and the token chain of
+// the weighted sum.  Four blocks read a split's rows, on one XCD (their linear
+// indexes differ by 2 max_splits, a multiple of 8 from 4 splits on), so three of
+// them find the rows in its L2; with all 8 heads in a block a cache of 8192 rows ran
+// 64 blocks and 5 serial rounds at 5000 tokens.
+constexpr int kSpanRounds = 8;
+constexpr int kSpanHeads = 2;
+constexpr int kSpanTokens = kSpanRounds * kRound;
+static_assert(kSpanHeads * kSpanRounds * kRound == kGqaThreads, "one weight a thread");
+
+__global__ __launch_bounds__(kGqaThreads)
+void gqa_span_kernel_bf16(const uint16_t* k_rows, const uint16_t* v_rows, const uint16_t* q_vec,
+                          const int32_t* kv_len_device, int64_t capacity, GqaArgs args) {
+    using T = Bf16;
+    GqaArgs a = args;
+    a.k = k_rows;
+    a.v = v_rows;
+    a.q = q_vec;
+    a.kv_len_device = kv_len_device;
+    a.capacity = capacity;
+    __shared__ __attribute__((aligned(16))) float s_v[kSpanTokens][kDim];
+    __shared__ __attribute__((aligned(16))) float s_sc[kSpanHeads][kSpanTokens];
+    __shared__ __attribute__((aligned(16))) float s_wt[kSpanHeads][kSpanTokens];
+    __shared__ float s_rm[kSpanHeads][kSpanRounds];  // maxima of the rounds
+    __shared__ float s_cr[kSpanHeads][kSpanRounds];  // rescales
+    __shared__ float s_M[kSpanHeads];
+    __shared__ float s_L[kSpanHeads];
+
+    const int g = blockIdx.y;
+    const int64_t s = blockIdx.x;
+    const int h0 = g * kHeadsPerGroup + kSpanHeads * blockIdx.z;  // first query head
+    const int tid = threadIdx.x;
+    const int gi = tid >> 4;
+    const int li = tid & 15;
+    const uint16_t* kbase = a.k + static_cast<int64_t>(g) * a.capacity * kDim + 8 * li;
+    const uint16_t* vbase = a.v + static_cast<int64_t>(g) * a.capacity * kDim + 8 * li;
+    const uint4 q0 = *reinterpret_cast<const uint4*>(a.q + h0 * kDim + 8 * li);
+    const uint4 q1 = *reinterpret_cast<const uint4*>(a.q + (h0 + 1) * kDim + 8 * li);
+
+    const int64_t L = read_kv_len(a);
+    const int64_t C = gqa_split_tokens(L, a.split_cap);
+    const int64_t nsplit = gqa_split_count(L, a.split_cap);
+    if (s >= nsplit) {
+        if (nsplit == 0 && s == 0 && tid < kSpanHeads * kDim) {
+            a.out[h0 * kDim + tid] = 0;  // empty cache
+        }
+        return;
+    }
+    const int64_t t0 = s * C;
+    const int64_t tend = t0 + C < L ? t0 + C : L;
+    float qa[8], qb[8];
+    unpack8<T>(q0, qa);
+    unpack8<T>(q1, qb);
+
+    // weights phase: half-wave (head wh, round wr), token wx; weighted sum: thread (head, dim)
+    const int wh = tid >> 8;
+    const int wr = (tid >> 5) & (kSpanRounds - 1);
+    const int wx = tid & (kRound - 1);
+    const int ph = tid >> 7;
+    const int pd = tid & (kDim - 1);
+    const bool sums = tid >= kSpanHeads * kDim && (tid & 127) == 0;  // thread 256 + 128 h sums head h's weights
+    float m_run = kNegInf;
+    float acc = 0.0f;
+    float lsum = 0.0f;
+
+#pragma unroll 1
+    for (int64_t b0 = t0; b0 < tend; b0 += kSpanTokens) {
+        const int left = static_cast<int>(tend - b0 < kSpanTokens ? tend - b0 : kSpanTokens);  // tokens of the span
+        const int rounds = (left + kRound - 1) / kRound;
+        uint4 kr[kSpanRounds], vr[kSpanRounds];
+#pragma unroll
+        for (int r = 0; r < kSpanRounds; ++r) {
+            load_row(kbase, vbase, b0 + kRound * r + gi, tend, kr[r], vr[r]);  // past the split: its last row
+        }
+#pragma unroll
+        for (int r = 0; r < kSpanRounds; ++r) {
+            if (r < rounds) {
+                float kf[8];
+                unpack8<T>(kr[r], kf);
+                float d0 = 0.0f;
+                float d1 = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    d0 = fmaf(qa[j], kf[j], d0);
+                    d1 = fmaf(qb[j], kf[j], d1);
+                }
+                // the butterfly's pairs at distances 8, 4, 2, 1; lanes 0..7 keep the first head
+                float z = (li < 8 ? d0 : d1) + row_ror<8>(li < 8 ? d1 : d0);
+                z = z + lane_xor4(z);
+                z = z + dpp<kDppXor2>(z);
+                z = z + dpp<kDppXor1>(z);
+                if ((li & 7) == 0) {
+                    s_sc[li >> 3][kRound * r + gi] = z * a.qk_scale_log2;
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < kSpanRounds; ++r) {
+            if (r < rounds) {
+                float vf[8];
+                unpack8<T>(vr[r], vf);
+                const bool live = kRound * r + gi < left;
+                float4* vrow = reinterpret_cast<float4*>(&s_v[kRound * r + gi][8 * li]);
+                vrow[0] = live ? make_float4(vf[0], vf[1], vf[2], vf[3]) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                vrow[1] = live ? make_float4(vf[4], vf[5], vf[6], vf[7]) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            }
+        }
+        __syncthreads();
+        const bool valid = kRound * wr + wx < left;
+        const float sc = s_sc[wh][kRound * wr + wx];
+        const float rm = span_max<kRound>(valid ? sc : kNegInf);
+        if (wx == 0) {
+            s_rm[wh][wr] = rm;
+        }
+        __syncthreads();
+        float m_prev = m_run;
+#pragma unroll
+        for (int r = 0; r < kSpanRounds; ++r) {
+            const float other = s_rm[wh][r];  // -inf past the span's rounds
+            m_prev = r < wr ? fmaxf(m_prev, other) : m_prev;
+            m_run = fmaxf(m_run, other);
+        }
+        const float m_new = fmaxf(m_prev, rm);
+        s_wt[wh][kRound * wr + wx] = valid ? exp2_fixed(sc - m_new) : 0.0f;
+        if (wx == 0) {
+            s_cr[wh][wr] = exp2_fixed(m_prev - m_new);
+        }
+        __syncthreads();
+        if (tid < kSpanHeads * kDim) {
+#pragma unroll 1
+            for (int r = 0; r < rounds; ++r) {
+                acc = acc * s_cr[ph][r];
+                const float* wp = &s_wt[ph][kRound * r];
+                const float* vp = &s_v[kRound * r][pd];
+                if (kRound * r + kRound <= left) {
+                    float v[kRound];
+                    float4 c[kRound / 4];
+#pragma unroll
+                    for (int x = 0; x < kRound; ++x) {
+                        v[x] = vp[x * kDim];
+                    }
+#pragma unroll
+                    for (int x = 0; x < kRound / 4; ++x) {
+                        c[x] = *reinterpret_cast<const float4*>(wp + 4 * x);
+                    }
+#pragma unroll
+                    for (int x = 0; x < kRound / 4; ++x) {
+                        acc = fmaf(c[x].x, v[4 * x], acc);
+                        acc = fmaf(c[x].y, v[4 * x + 1], acc);
+                        acc = fmaf(c[x].z, v[4 * x + 2], acc);
+                        acc = fmaf(c[x].w, v[4 * x + 3], acc);
+                    }
+                } else {
+                    const int nq = (left - kRound * r + 3) & ~3;  // whole quads: staged zeros past the end
+#pragma unroll 1
+                    for (int x = 0; x < nq; x += 4) {
+                        const float4 c = *reinterpret_cast<const float4*>(wp + x);
+                        acc = fmaf(c.x, vp[x * kDim], acc);
+                        acc = fmaf(c.y, vp[(x + 1) * kDim], acc);
+                        acc = fmaf(c.z, vp[(x + 2) * kDim], acc);
+                        acc = fmaf(c.w, vp[(x + 3) * kDim], acc);
+                    }
+                }
+            }
+        } else if (sums) {
+            const int h = ph - kSpanHeads;
+#pragma unroll 1
+            for (int r = 0; r < rounds; ++r) {
+                lsum = lsum * s_cr[h][r];
+                float4 c[kRound / 4];
+#pragma unroll
+                for (int x = 0; x < kRound / 4; ++x) {
+                    c[x] = *reinterpret_cast<const float4*>(&s_wt[h][kRound * r + 4 * x]);
+                }
+#pragma unroll
+                for (int x = 0; x < kRound / 4; ++x) {  // weights past the end are zero: they leave the sum as it is
+                    lsum = lsum + c[x].x;
+                    lsum = lsum + c[x].y;
+                    lsum = lsum + c[x].z;
+                    lsum = lsum + c[x].w;
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if (sums) {
+        s_L[ph - kSpanHeads] = lsum;
+    }
+    if (wr == 0 && wx == 0) {
+        s_M[wh] = m_run;
+    }
+    __syncthreads();
+    if (tid >= kSpanHeads * kDim) {
+        return;
+    }
+    if (nsplit == 1) {
+        // single split: the general merge with weight exp2(M - M) = 1
+        const float w = exp2_fixed(s_M[ph] - s_M[ph]);
+        const float lt = fmaf(s_L[ph], w, 0.0f);
+        a.out[(h0 + ph) * kDim + pd] = T::store(fmaf(acc, w, 0.0f) * (1.0f / lt));
+        return;
+    }
+    float* dst = a.partials + ((h0 + ph) * a.max_splits + s) * kPartialStride;
+    dst[2 + pd] = acc;
+    if (pd == 0) {
+        *reinterpret_cast<float2*>(dst) = make_float2(s_M[ph], s_L[ph]);
+    }
+}
+
 // grid (16 query heads, 8 slices of 16 dims), 256 threads.  Thread t loads
 // dim t%16 of the slice for splits t/16, t/16 + 16, ... (16 lanes read one
 // 64-byte run of a split row), all in flight before the first LDS store, and
@@ -959,7 +1176,13 @@ hipError_t launch_gqa_decode(Act act, const GqaArgs& a, hipStream_t stream) {
         return hipErrorInvalidValue;
     }
     const dim3 grid(static_cast<unsigned>(a.max_splits), 2);
-    if (act == Act::kBf16) {
+    if (a.spans) {
+        if (act != Act::kBf16 || a.ticket_max != 1 || a.defer_max != 0) {
+            return hipErrorInvalidValue;
+        }
+        hipLaunchKernelGGL(gqa_span_kernel_bf16, dim3(grid.x, 2, kHeadsPerGroup / kSpanHeads), dim3(kGqaThreads), 0, stream,
+                           a.k, a.v, a.q, a.kv_len_device, a.capacity, a);
+    } else if (act == Act::kBf16) {
         hipLaunchKernelGGL(gqa_partial_kernel_bf16, grid, dim3(kGqaThreads), 0, stream, a.k, a.v, a.q,
                            a.kv_len_device, a.capacity, a);
     } else {

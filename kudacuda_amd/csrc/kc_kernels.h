@@ -261,6 +261,9 @@ struct GqaArgs {
     // splits (8 splits: 7.5 vs 8.0 us, 16: 8.3 vs 8.5) and loses at 32 (11.1
     // vs 8.9 us).
     int64_t ticket_max = 16;
+    // bf16 round path with defer_max 0 and ticket_max 1: the kernel that works on a
+    // split's rounds side by side, two heads a block (the same bits)
+    bool spans = false;
     float qk_scale_log2 = 0.0f;    // scale * log2(e)
     bool mfma = false;             // split plan of the matrix-core tactic (gqa_mfma_split_tokens)
     int64_t mfma_quantum = kGqaMfmaQuantum;  // its split unit: 64 (2-wave blocks) or 128 (4-wave blocks)

@@ -454,8 +454,9 @@ struct Model {
     std::array<uint64_t, KUDACUDA_QWEN2_MODEL_FIELDS> g{};
     hipGraph_t graph = nullptr;
     // the captured step in each of its forms (index = form, see model_op);
-    // forms 1 .. step_defer_cap always, form 0 when the cache can need it
-    std::array<hipGraphExec_t, kGqaMaxDefer + 1> execs{};
+    // forms 1 .. step_defer_cap always, form 0 and kSpanStepForm when the cache
+    // can need them
+    std::array<hipGraphExec_t, kGqaMaxDefer + 2> execs{};
     // the step (control[0]) the next launch runs at, as far as the host
     // knows (-1: unknown); only picks among the step forms, which compute
     // the same results
@@ -484,18 +485,27 @@ int64_t step_defer_cap(const Model& m) {
 // before positions were tracked.
 constexpr int64_t kUnknownStepForm = 6;
 
+// Form 0 with gqa_span_kernel_bf16 in place of the one-round-at-a-time kernel,
+// for lengths whose splits have more than one round (over 1024 cached tokens).
+// Whole step, us, that kernel -> this form: 1500 tokens 1143 -> 1114, 2500 1203 ->
+// 1137, 5000 1313 -> 1192, 8000 1519 -> 1274; with one round a split (600 tokens
+// 1081 -> 1096) it loses, its four blocks a split and no rows requested before
+// kv_len is known.
+constexpr int kSpanStepForm = kGqaMaxDefer + 1;
+
 // form (ops 1 and 2 only): k = 1 .. step_defer_cap -- attention leaves up to
 // k splits to o_proj, whose merge prologue requests exactly k split slots,
 // and merges more by its own ticket (no merge launch in the graph); -1: the
 // unknown-position form, kUnknownStepForm (or the cap, if smaller); 0 -- the
 // form for caches whose split count exceeds the cap:
 // attention's partials all go to gqa_merge_kernel (one more launch, parallel
-// over heads and dims) and o_proj reads the merged vector as a plain GEMV.
+// over heads and dims) and o_proj reads the merged vector as a plain GEMV;
+// kSpanStepForm -- form 0 for splits of several rounds.
 // Every form merges by the same rule in the same order: identical results at
 // any length, only the time differs.
 hipError_t model_op(const Model& m, int op, int64_t layer, bool bookkeeping, hipStream_t stream,
                     int form = -1) {
-    const bool long_ctx = form == 0;
+    const bool long_ctx = form == 0 || form == kSpanStepForm;
     const int64_t cap = step_defer_cap(m);
     const int64_t want = form < 0 ? kUnknownStepForm : form;
     const int64_t defer = want < cap ? want : cap;
@@ -549,6 +559,7 @@ hipError_t model_op(const Model& m, int op, int64_t layer, bool bookkeeping, hip
             if (long_ctx) {
                 a.defer_max = 0;   // gqa_merge_kernel merges every split count above one
                 a.ticket_max = 1;
+                a.spans = form == kSpanStepForm;
             } else {
                 a.defer_max = defer;  // o_proj merges these
                 // the rest by ticket: a merge kernel would be one more graph
@@ -815,7 +826,8 @@ hipError_t model_prefill(const Model& m, uint8_t* ws, int64_t start, int64_t cou
 }
 
 // The fastest form for the step at `step` (kv_len step + 1): the split
-// count itself while o_proj merges it, form 0 past the cap, kUnknownStepForm
+// count itself while o_proj merges it, past the cap form 0 (one round a split) or
+// kSpanStepForm (more), kUnknownStepForm
 // (or the cap, if smaller) when the step is unknown.
 int step_form(const Model& m, int64_t step) {
     const int64_t cap = step_defer_cap(m);
@@ -826,11 +838,18 @@ int step_form(const Model& m, int64_t step) {
     set_gqa_plan(plan, m.capacity, kGqaStepSplits);
     const int64_t kv_len = step + 1 < m.capacity ? step + 1 : m.capacity;
     const int64_t nsplit = gqa_split_count(kv_len, plan.split_cap);
-    return nsplit > cap ? 0 : static_cast<int>(nsplit < 1 ? 1 : nsplit);
+    if (nsplit > cap) {
+        return gqa_split_tokens(kv_len, plan.split_cap) > kGqaRoundTokens ? kSpanStepForm : 0;
+    }
+    return static_cast<int>(nsplit < 1 ? 1 : nsplit);
 }
 
-// Whether a cache of the model's capacity can need form 0 at all.
-bool long_form_possible(const Model& m) { return step_form(m, m.capacity - 1) == 0; }
+// Whether a cache of the model's capacity can need a form at all (the forms of
+// shorter lengths are needed with those of longer ones).
+bool form_possible(const Model& m, int form) {
+    const int longest = step_form(m, m.capacity - 1);
+    return form == 0 ? longest == 0 || longest == kSpanStepForm : form != kSpanStepForm || longest == form;
+}
 
 hipError_t model_step(const Model& m, hipStream_t stream, int form = -1) {
     for (int64_t layer = 0; layer < m.num_layers; ++layer) {
@@ -1669,10 +1688,13 @@ int kudacuda_qwen2_model_capture(void* raw_model, uint64_t stream) {
     };
     drop_all();
     hipStream_t s = as_stream(stream);
-    // forms 1 .. cap always (the split count a step can leave to o_proj),
-    // form 0 when this cache can exceed the cap
+    // forms 1 .. cap always (the split count a step can leave to o_proj), the
+    // long ones when this cache can exceed the cap
     const int cap = static_cast<int>(kc::step_defer_cap(*m));
-    for (int form = kc::long_form_possible(*m) ? 0 : 1; form <= cap; ++form) {
+    for (int form = 0; form <= kc::kSpanStepForm; ++form) {
+        if ((form > cap && form != kc::kSpanStepForm) || !kc::form_possible(*m, form)) {
+            continue;
+        }
         hipError_t status = hipStreamBeginCapture(s, hipStreamCaptureModeGlobal);
         if (status != hipSuccess) {
             drop_all();
