@@ -546,9 +546,13 @@ hipError_t launch_few_shape(const Nf4GemmArgs& a, hipStream_t stream) {
         return one ? launch_few<EPI, 2, 4, 1>(a, splits, stream) : launch_few<EPI, 2, 4, 2>(a, splits, stream);
     }
     // a short k: as many fragments a block as make one round of blocks, unsplit (q of 64
-    // tokens 8.3 us in 64 blocks, 9.2 split in four); very few blocks (k, v) are split
+    // tokens 8.3 us in 64 blocks, 9.2 split in four); very few blocks (k, v) are split.
+    // A row norm needs a second launch either way, so o_proj splits over the whole
+    // chip and norms in its reduce (prefill of 9 layers, us, unsplit -> split: 1 token
+    // 505 -> 487, 16 511 -> 490, 48 629 -> 594, 64 643 -> 616)
     if (units * tiles <= kBlocks) {
-        const int64_t splits = units * tiles < 64 ? 64 / (units * tiles) : 1;
+        const int64_t fill = EPI == GemmEpi::kResidualNorm ? kBlocks : 64;
+        const int64_t splits = units * tiles < fill ? fill / (units * tiles) : 1;
         return one ? launch_few<EPI, 1, 4, 1>(a, splits, stream) : launch_few<EPI, 1, 4, 2>(a, splits, stream);
     }
     if ((units + 1) / 2 * tiles <= kBlocks) {
