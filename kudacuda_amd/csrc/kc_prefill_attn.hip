@@ -10,24 +10,29 @@
 // the softmax needs one lane-half exchange for the maximum and none for the sum
 // before the end.  Those 32 lie in exactly the B layout that P needs for
 // out^T = V^T P^T if V^T's keys are stored in that order, so the weights never
-// leave their lane.  They enter as two MFMAs, bf16 halves of the fp32 weight and
-// of its remainder (16 bits of every weight; the decode kernel's scheme).
+// leave their lane.  They enter as three MFMAs, bf16 parts of 8 bits each whose
+// sum is the fp32 weight.  Error before the output's rounding, against 64 bits
+// (2-norm, random rows; the row kernel's fp32 sums / this / with two parts): 300
+// tokens 1.9e-7 / 1.1e-7 / 1.8e-6, 512 after 1024 8.2e-7 / 2.0e-7 / 2.2e-6, 1999
+// 3.9e-7 / 1.7e-7 / 1.9e-6; two parts take 46 us a layer at 1999 tokens, three 54.
+// The hardware's exp2 (at most 0.78 ulp off below 0, exp2_fixed 0.87) leaves these
+// figures as they are; exp2_fixed in its place takes 95 us.
 // V is transposed on its way into LDS (4 keys x 8 dims a thread, byte permutes);
 // K rows are swizzled by 16-byte piece; the next window's rows are requested
 // while one is computed.
 //
 // Operands are read from LDS a step ahead of their MFMAs and the weights of 16
 // keys are formed between the MFMAs of the 16 before, held there by scheduling
-// barriers (left to the compiler each read stalled its own MFMA: 1999 tokens 67
-// -> 43 us).  A wave of the window takes 48 MFMAs and about as long in fp32
-// arithmetic; two waves a SIMD overlap the two.  Work grows with the position:
+// barriers (left to the compiler each read stalled its own MFMA; with two parts
+// 1999 tokens 67 -> 43 us).  A wave of the window takes 64 MFMAs and about as long
+// in fp32 arithmetic; two waves a SIMD overlap the two.  Work grows with the position:
 // blocks are ordered heavy to light, then light to heavy, so the two that share
 // a CU add up alike.
 //
 // Few tokens over a long cache split the windows over blocks (S) and merge
 // partials in a second kernel.  Measured per layer (MI355X, us; before = one
-// block per query row, fp32 dot products): 1999 tokens 847 -> 43, 512 after 1024
-// 288 -> 25 + 5 (merge), 10 after 1961 about 70 -> 8 + 4.
+// block per query row, fp32 dot products): 1999 tokens 847 -> 54, 512 after 1024
+// 288 -> 29 + 5 (merge), 10 after 1961 about 70 -> 8 + 4.
 #include "kc_device.h"
 #include "kc_kernels.h"
 
@@ -319,9 +324,10 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_mfma_kernel(PrefillA
             }
             m_run = m_new;
         }
-        // weights of 16 keys (step n: scores 8 (n % 2) .. + 7 of tile n / 2) as a
-        // high and a low bf16 half, pair by pair
-        uint32_t hi[2][4], lo[2][4];
+        // weights of 16 keys (step n: scores 8 (n % 2) .. + 7 of tile n / 2) as
+        // three bf16 parts, pair by pair: 8 bits each, their sum is the fp32
+        // weight exactly (both remainders are exact)
+        uint32_t hi[2][4], mid[2][4], lo[2][4];
         auto weights = [&](int n, int e) __attribute__((always_inline)) {
             const float p0 =
                 __builtin_amdgcn_exp2f(fmaf(sc[n / 2][8 * (n % 2) + 2 * e], a.qk_scale_log2, -m_sub));
@@ -330,7 +336,11 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_mfma_kernel(PrefillA
             l_run += p0 + p1;
             const uint32_t h = pack2(p0, p1);
             hi[n & 1][e] = h;
-            lo[n & 1][e] = pack2(p0 - __uint_as_float(h << 16), p1 - __uint_as_float(h & 0xffff0000u));
+            const float r0 = p0 - __uint_as_float(h << 16);
+            const float r1 = p1 - __uint_as_float(h & 0xffff0000u);
+            const uint32_t m = pack2(r0, r1);
+            mid[n & 1][e] = m;
+            lo[n & 1][e] = pack2(r0 - __uint_as_float(m << 16), r1 - __uint_as_float(m & 0xffff0000u));
         };
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -342,10 +352,13 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_mfma_kernel(PrefillA
 #pragma unroll
         for (int n = 0; n < 4; ++n) {
             const bf16x8 ph = __builtin_bit_cast(bf16x8, make_uint4(hi[n & 1][0], hi[n & 1][1], hi[n & 1][2], hi[n & 1][3]));
+            const bf16x8 pm =
+                __builtin_bit_cast(bf16x8, make_uint4(mid[n & 1][0], mid[n & 1][1], mid[n & 1][2], mid[n & 1][3]));
             const bf16x8 pl = __builtin_bit_cast(bf16x8, make_uint4(lo[n & 1][0], lo[n & 1][1], lo[n & 1][2], lo[n & 1][3]));
 #pragma unroll
             for (int dt = 0; dt < 4; ++dt) {
                 acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vf[dt]), ph, acc[dt], 0, 0, 0);
+                acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vf[dt]), pm, acc[dt], 0, 0, 0);
                 acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vf[dt]), pl, acc[dt], 0, 0, 0);
                 if (n < 3) {
                     weights(n + 1, dt);
@@ -355,7 +368,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_mfma_kernel(PrefillA
             }
         }
     }
-    // Zero weights (hidden keys, the low half of a weight) times an infinity or
+    // Zero weights (hidden keys, the lower parts of a weight) times an infinity or
     // NaN of V are NaN: a block whose result is not finite starts again, key by
     // key in fp32 with hidden keys left out.
     {
@@ -377,7 +390,12 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_mfma_kernel(PrefillA
                      static_cast<int64_t>(w_end) * kWindowKeys);
         return;
     }
-    // the K-groups' results meet in group 0
+    // the K-groups' results meet in group 0; the lane's column is formed again
+    // (kept over the loop, which uses every register, its values spilled)
+    const int fl = static_cast<int>(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)));
+    const int fq = fl >> 5;
+    const int ftok = row0 + 4 * cg + fl % 32 / kHeads;
+    const int fhead = g * kHeads + fl % kHeads;
     l_run = sum_halves(l_run);
     float* const s_acc = reinterpret_cast<float*>(smem);
     float* const s_ml = s_acc + 2 * 64 * 64;
@@ -386,19 +404,19 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_mfma_kernel(PrefillA
         for (int dt = 0; dt < 4; ++dt) {
 #pragma unroll
             for (int i4 = 0; i4 < 4; ++i4) {
-                reinterpret_cast<float4*>(s_acc)[(cg * 16 + dt * 4 + i4) * 64 + lane] =
+                reinterpret_cast<float4*>(s_acc)[(cg * 16 + dt * 4 + i4) * 64 + fl] =
                     make_float4(acc[dt][4 * i4], acc[dt][4 * i4 + 1], acc[dt][4 * i4 + 2], acc[dt][4 * i4 + 3]);
             }
         }
-        s_ml[cg * 128 + 2 * lane] = m_run;
-        s_ml[cg * 128 + 2 * lane + 1] = l_run;
+        s_ml[cg * 128 + 2 * fl] = m_run;
+        s_ml[cg * 128 + 2 * fl + 1] = l_run;
     }
     __syncthreads();
     if (kg == 1) {
         return;
     }
-    const float m1 = s_ml[cg * 128 + 2 * lane];
-    const float l1 = s_ml[cg * 128 + 2 * lane + 1];
+    const float m1 = s_ml[cg * 128 + 2 * fl];
+    const float l1 = s_ml[cg * 128 + 2 * fl + 1];
     const float m_all = fmaxf(m_run, m1);
     const float m_sub = m_all == kNegInf ? 0.0f : m_all;
     const float c0 = __builtin_amdgcn_exp2f(m_run - m_sub);
@@ -408,7 +426,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_mfma_kernel(PrefillA
     for (int dt = 0; dt < 4; ++dt) {
 #pragma unroll
         for (int i4 = 0; i4 < 4; ++i4) {
-            const float4 v = reinterpret_cast<const float4*>(s_acc)[(cg * 16 + dt * 4 + i4) * 64 + lane];
+            const float4 v = reinterpret_cast<const float4*>(s_acc)[(cg * 16 + dt * 4 + i4) * 64 + fl];
             acc[dt][4 * i4] = acc[dt][4 * i4] * c0 + v.x * c1;
             acc[dt][4 * i4 + 1] = acc[dt][4 * i4 + 1] * c0 + v.y * c1;
             acc[dt][4 * i4 + 2] = acc[dt][4 * i4 + 2] * c0 + v.z * c1;
@@ -416,39 +434,38 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_mfma_kernel(PrefillA
         }
     }
     if (S > 1) {
-        if (tok < M) {
-            const int64_t at = (static_cast<int64_t>(row) * 16 + head) * S + split;
+        if (ftok < M) {
+            const int64_t at = (static_cast<int64_t>(ftok) * 16 + fhead) * S + split;
             float* dst = a.partials + at * kDim;
 #pragma unroll
             for (int dt = 0; dt < 4; ++dt) {
 #pragma unroll
                 for (int i4 = 0; i4 < 4; ++i4) {
-                    *reinterpret_cast<float4*>(dst + 32 * dt + 8 * i4 + 4 * q) =
+                    *reinterpret_cast<float4*>(dst + 32 * dt + 8 * i4 + 4 * fq) =
                         make_float4(acc[dt][4 * i4], acc[dt][4 * i4 + 1], acc[dt][4 * i4 + 2], acc[dt][4 * i4 + 3]);
                 }
             }
-            if (q == 0) {
+            if (fq == 0) {
                 *reinterpret_cast<float2*>(a.partials + a.m * 16 * S * kDim + 2 * at) = make_float2(m_all, l_all);
             }
         }
         return;
     }
-    const float inv = 1.0f / l_all;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) {
         uint32_t h[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            h[e] = pack2(acc[dt][2 * e] * inv, acc[dt][2 * e + 1] * inv);
+            h[e] = pack2(acc[dt][2 * e] / l_all, acc[dt][2 * e + 1] / l_all);
         }
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             // lane halves exchange so that each holds 8 consecutive dims
             const auto s0 = __builtin_amdgcn_permlane32_swap(h[4 * j], h[4 * j + 2], false, false);
             const auto s1 = __builtin_amdgcn_permlane32_swap(h[4 * j + 1], h[4 * j + 3], false, false);
-            if (tok < M) {
-                *reinterpret_cast<uint4*>(a.out + static_cast<int64_t>(row) * 2048 + head * kDim + 32 * dt + 16 * j +
-                                          8 * q) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
+            if (ftok < M) {
+                *reinterpret_cast<uint4*>(a.out + static_cast<int64_t>(ftok) * 2048 + fhead * kDim + 32 * dt + 16 * j +
+                                          8 * fq) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
             }
         }
     }
@@ -536,9 +553,8 @@ __global__ __launch_bounds__(256) void prefill_attention_merge_kernel(PrefillAtt
             v.w = fmaf(p.w, co, v.w);
         }
     }
-    const float inv = 1.0f / l;
     *reinterpret_cast<uint2*>(a.out + row * 2048 + head * kDim + d) =
-        make_uint2(pack2(v.x * inv, v.y * inv), pack2(v.z * inv, v.w * inv));
+        make_uint2(pack2(v.x / l, v.y / l), pack2(v.z / l, v.w / l));
 }
 
 }  // namespace
