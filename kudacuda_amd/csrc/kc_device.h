@@ -130,6 +130,29 @@ __device__ __forceinline__ float silu_fixed(float g) {
     return g / (1.0f + e);
 }
 
+// The same for |g| < kSiluNear (or NaN), without exp2_fixed's two branches and
+// with one correction of g * rcp in place of the full division: 18 instructions
+// instead of 32.  Compared on gfx950 with silu_fixed for every float in that
+// range: no bit differs.
+constexpr float kSiluNear = 86.0f;
+__device__ __forceinline__ float silu_near(float g) {
+    const float y = g * -kLog2e;
+    const float n = rintf(y);
+    const float f = y - n;
+    float p = 0x1.ffcbfcp-17f;
+    p = fmaf(p, f, 0x1.430912p-13f);
+    p = fmaf(p, f, 0x1.5d87fep-10f);
+    p = fmaf(p, f, 0x1.3b2ab6p-7f);
+    p = fmaf(p, f, 0x1.c6b08ep-5f);
+    p = fmaf(p, f, 0x1.ebfbe0p-3f);
+    p = fmaf(p, f, 0x1.62e430p-1f);
+    p = fmaf(p, f, 1.0f);
+    const float d = 1.0f + ldexpf(p, static_cast<int>(n));
+    const float r = __builtin_amdgcn_rcpf(d);
+    const float q = g * r;
+    return fmaf(-fmaf(d, q, -g), r, q);
+}
+
 // ---------------------------------------------------------------- reductions
 // DPP row rotation (row_ror:N, rotate within each row of 16 lanes).
 template <int N>

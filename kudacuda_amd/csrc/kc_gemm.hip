@@ -34,7 +34,8 @@
 // time), and a block's prologue (table fill, first operands) and epilogue hide
 // only behind another block of the CU.  Hence the shapes in launch_shape().
 // Measured at 1999 tokens (MI355X, us per call; before = 64-token launches):
-// gate/up SwiGLU 621 -> 201 (896 TFLOP/s), down 519 -> 112 (807), q/k/v rows
+// gate/up SwiGLU 621 -> 207 (869 TFLOP/s; silu by hardware exp2 and reciprocal, up
+// to 2.7 ulp off where silu_fixed is 2.0, 201; by silu_fixed itself 215), down 519 -> 112 (807), q/k/v rows
 // 340 -> 43 (486); at 128 tokens 46 -> 26, 36 -> 23, 24 -> 17.
 #include "kc_device.h"
 #include "kc_kernels.h"
@@ -66,11 +67,6 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
 }
 __device__ __forceinline__ float lo_f32(uint32_t v) { return __uint_as_float(v << 16); }
 __device__ __forceinline__ float hi_f32(uint32_t v) { return __uint_as_float(v & 0xffff0000u); }
-
-// silu(g) by the hardware's exp2 and reciprocal (1 ulp each).
-__device__ __forceinline__ float silu_fast(float g) {
-    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -kLog2e));
-}
 
 // A fragment's packed column pairs of one token (h[2 i4 + e]: columns 8 i4 +
 // 4 q + 2 e and the next) as 8 consecutive columns a lane: o[j] holds columns
@@ -429,10 +425,23 @@ __global__ __launch_bounds__(64 * WN * WK, WN * RF > 4 || WK * RF < 4 ? 2 : 1) v
         for (int t = 0; t < kFin; ++t) {
             const int m = mf + 32 * t + r;
             uint32_t h[8];
+            float far = 0.0f;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                h[i] = pack2(silu_fast(fin[0][t][2 * i]) * fin[1][t][2 * i],
-                             silu_fast(fin[0][t][2 * i + 1]) * fin[1][t][2 * i + 1]);
+            for (int i = 0; i < 16; ++i) {
+                far = fmaxf(far, fabsf(fin[0][t][i]));
+            }
+            if (__any(far >= kSiluNear)) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    h[i] = pack2(silu_fixed(fin[0][t][2 * i]) * fin[1][t][2 * i],
+                                 silu_fixed(fin[0][t][2 * i + 1]) * fin[1][t][2 * i + 1]);
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    h[i] = pack2(silu_near(fin[0][t][2 * i]) * fin[1][t][2 * i],
+                                 silu_near(fin[0][t][2 * i + 1]) * fin[1][t][2 * i + 1]);
+                }
             }
             uint4 o[2];
             rows16(h, o);
@@ -602,7 +611,7 @@ hipError_t launch_tile(const Nf4GemmArgs& a, int64_t blocks, int64_t min_split, 
 //   down   wide      31.5  38.6  56.5  92.3   163
 //          square    26.2  31.4  42.4  68.8   114
 //          low       23.1  30.7  48.9  80.7   155
-//   gate/up wide     36.4  37.9  62.7   108   201
+//   gate/up wide     36.4  39.1  65.7   112   207
 //           pair     25.7  47.4  70.8   144   274
 // One fragment a wave cannot hold a gate/up or rotary pair: those epilogues run
 // in the split reduce, or in the wide and pair shapes.

@@ -70,6 +70,42 @@ def test_nf4_gemm_swiglu_of_many_tokens_matches_fp64(torch_gpu, native, stream, 
     _close(host(out).reshape(m, n), want)
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (64, 8192, 256),     # the few-token kernel
+    (500, 3968, 128),    # pair blocks
+    (300, 11008, 128),   # wide blocks
+])
+def test_swiglu_of_exact_sums_is_the_oracles(torch_gpu, native, stream, m, n, k):
+    """Each token has two elements, powers of two 9 bits apart: the sums are exact,
+    so every output is bf16(silu(gate) * up) of the oracle's fp32 silu to the bit,
+    in every kernel (a silu 1 ulp off moves about 1 output in 80,000).  The gates
+    of the last token are large enough for either branch of the silu."""
+
+    torch = torch_gpu
+    rng = np.random.default_rng([SEED, 8, m, n, k])
+    print(f"nf4_gemm_swiglu of two-element tokens m={m} n={n} k={k}", flush=True)
+    gp, ga, gw = _weights(rng, n, k, std=0.06)
+    up, ua, uw = _weights(rng, n, k, std=0.06)
+    x = np.zeros((m, k), np.float32)
+    scale = 2.0 ** rng.integers(0, 6, m)
+    scale[-1] = 2.0 ** 11
+    at = rng.integers(0, k // 2, m)
+    x[np.arange(m), at] = scale
+    x[np.arange(m), at + k // 2] = scale * 2.0 ** -9
+    gate, upv = (x.astype(np.float64) @ w.T for w in (gw, uw))
+    for sums in (gate, upv):
+        assert np.array_equal(sums, sums.astype(np.float32))
+    assert np.abs(gate[-1]).max() > 128
+    out = empty(torch, m * n, "u16")
+    bufs = [dev(torch, t) for t in (O.f32_to_bf16(x), gp, ga, up, ua)]
+    native.call("kudacuda_nf4_gemm_swiglu_bf16", *[p(b) for b in bufs], p(out), m, k, n, 64, stream.cuda_stream)
+    stream.synchronize()
+    got = O.bf16_to_f32(host(out).reshape(m, n))
+    want = O.bf16_to_f32(O.f32_to_bf16(O.silu(gate.astype(np.float32)) * upv.astype(np.float32)))
+    print(f"{int(np.count_nonzero(got != want))} of {got.size} differ", flush=True)
+    assert np.array_equal(got, want)
+
+
 @pytest.mark.parametrize("count", [200, 301, 900, 1700])
 def test_prefill_rows_equal_those_of_64_token_parts(torch_gpu, native, count):
     """One layer: a long prompt at once (q, k, v in low, square, pair and wide
