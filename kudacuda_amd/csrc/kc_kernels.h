@@ -261,13 +261,16 @@ struct GqaArgs {
     // splits (8 splits: 7.5 vs 8.0 us, 16: 8.3 vs 8.5) and loses at 32 (11.1
     // vs 8.9 us).
     int64_t ticket_max = 16;
+    float qk_scale_log2 = 0.0f;    // scale * log2(e)
+    bool mfma = false;             // split plan of the matrix-core tactic (gqa_mfma_split_tokens)
     // bf16 round path with defer_max 0 and ticket_max 1: the kernel that works on a
     // split's rounds side by side, two heads a block (the same bits)
     bool spans = false;
-    float qk_scale_log2 = 0.0f;    // scale * log2(e)
-    bool mfma = false;             // split plan of the matrix-core tactic (gqa_mfma_split_tokens)
-    int64_t mfma_quantum = kGqaMfmaQuantum;  // its split unit: 64 (2-wave blocks) or 128 (4-wave blocks)
+    int64_t mfma_quantum = kGqaMfmaQuantum;  // the matrix-core split unit: 64 (2-wave blocks) or 128 (4-wave blocks)
 };
+// Two 64-byte lines of kernel arguments: every GQA kernel waits for the line its
+// split plan is in (a third line cost the direct call over 30000 tokens 0.2 of 16 us).
+static_assert(sizeof(GqaArgs) == 128, "two lines of kernel arguments");
 hipError_t launch_gqa_decode(Act act, const GqaArgs& args, hipStream_t stream);
 // Matrix-core tactic (v_mfma_f32_16x16x32_{bf16,f16} for q.K and P.V, the
 // weights P as a hi + lo pair of 16-bit values): partial kernel with
