@@ -32,13 +32,13 @@
 // What bounds it: two waves a SIMD are needed to keep the matrix core busy (a
 // wave alone issues its ~7 instructions per MFMA in about twice the MFMA's
 // time), and a block's prologue (table fill, first operands) and epilogue hide
-// only behind another block of the CU.  Hence the shapes in launch_shape().
+// only behind another block of the CU.  Hence the shapes in kc_gemm_plan.h.
 // Measured at 1999 tokens (MI355X, us per call; before = 64-token launches):
 // gate/up SwiGLU 621 -> 207 (869 TFLOP/s; silu by hardware exp2 and reciprocal, up
-// to 2.7 ulp off where silu_fixed is 2.0, 201; by silu_fixed itself 215), down 519 -> 112 (807), q/k/v rows
-// 340 -> 43 (486); at 128 tokens 46 -> 26, 36 -> 23, 24 -> 17.
+// to 2.7 ulp off where silu_fixed is 2.0, 201; by silu_fixed itself about 215), down
+// 519 -> 112 (807), q/k/v rows 340 -> 43 (486).
 #include "kc_device.h"
-#include "kc_kernels.h"
+#include "kc_gemm_plan.h"
 
 namespace kc {
 namespace {
@@ -418,8 +418,8 @@ __global__ __launch_bounds__(64 * WN * WK, WN * RF > 4 || WK * RF < 4 ? 2 : 1) v
         }
         return;
     }
-    if constexpr (RF == 1 && (EPI == GemmEpi::kSwiGlu || EPI == GemmEpi::kQkvRope)) {
-        return;  // split only: their epilogues need both fragments
+    if constexpr (RF == 1 && EPI == GemmEpi::kQkvRope) {
+        return;  // split only: the rotation needs both fragments
     } else if constexpr (EPI == GemmEpi::kSwiGlu) {
 #pragma unroll
         for (int t = 0; t < kFin; ++t) {
@@ -551,29 +551,12 @@ __global__ __launch_bounds__(64 * WN * WK, WN * RF > 4 || WK * RF < 4 ? 2 : 1) v
     }
 }
 
-// K is split so that the launch has about `blocks` blocks, as far as the partial
-// tiles fit a.partials; refused when that leaves fewer than min_split splits.
 template <GemmEpi EPI, int WN, int WK, int RF, int NT>
-hipError_t launch_tile(const Nf4GemmArgs& a, int64_t blocks, int64_t min_split, hipStream_t stream) {
+hipError_t launch_tile(const Nf4GemmArgs& a, int64_t S, hipStream_t stream) {
     constexpr bool kPairs = EPI == GemmEpi::kSwiGlu && RF == 2;  // gate and up rows share a tile
     constexpr int64_t kRows = (kPairs ? 32 : 32 * RF) * WN;
-    constexpr int NF = EPI == GemmEpi::kSwiGlu ? 2 : 1;
-    const int64_t m_tiles = (a.m + 32 * NT - 1) / (32 * NT);
-    const int64_t n_tiles = (a.n + kRows - 1) / kRows;
-    const int64_t windows = a.k / (kWindow * WK);
-    int64_t S = a.partials == nullptr ? 1 : blocks / (m_tiles * n_tiles);
-    S = S < windows ? S : windows;
-    while (S > 1 && NF * S * a.m * a.n > a.partial_floats) {
-        --S;
-    }
-    if (S > 1) {
-        const int64_t per_split = (windows + S - 1) / S;
-        S = (windows + per_split - 1) / per_split;  // no empty split
-    }
-    S = S > 1 ? S : 1;
-    if (S < min_split) {
-        return hipErrorInvalidValue;
-    }
+    const int64_t m_tiles = gemm_ceil(a.m, 32 * NT);
+    const int64_t n_tiles = gemm_ceil(a.n, kRows);
     hipLaunchKernelGGL((nf4_tile_gemm_kernel<EPI, WN, WK, RF, NT>), dim3(static_cast<unsigned>(m_tiles * n_tiles * S)),
                        dim3(64 * WN * WK), 0, stream, a, static_cast<int>(m_tiles), static_cast<int>(n_tiles),
                        static_cast<int>(S));
@@ -596,102 +579,44 @@ hipError_t launch_tile(const Nf4GemmArgs& a, int64_t blocks, int64_t min_split, 
     return hipSuccess;
 }
 
-// Block shapes (rows x tokens), each with the number of blocks that fill the
-// chip, measured on one box (us per call, q = 2560 rows of k 2048, down = 2048
-// rows of k 11008, gate/up = 2 x 11008 rows of k 2048):
-//   wide   256 x 128, 4 waves, two blocks a CU
-//   square 128 x 128, 8 waves of one fragment in two K-groups, one block a CU
-//   pair   128 x 128, 4 waves of two fragments in two K-groups, one block a CU
-//   low    128 x 64, 8 waves in two K-groups, one block a CU
-//   tokens            128   256   512  1024  1999
-//   q      wide      24.2  26.4  31.2  41.8  43.1
-//          square    19.9  22.9  25.6  26.5  49.1
-//          pair      21.4  24.2  27.3  28.3  52.7
-//          low       16.9  18.7  18.7  31.1  48.3
-//   down   wide      31.5  38.6  56.5  92.3   163
-//          square    26.2  31.4  42.4  68.8   114
-//          low       23.1  30.7  48.9  80.7   155
-//   gate/up wide     36.4  39.1  65.7   112   207
-//           pair     25.7  47.4  70.8   144   274
-// One fragment a wave cannot hold a gate/up or rotary pair: those epilogues run
-// in the split reduce, or in the wide and pair shapes.
+// The shapes that gemm_tile_plan() gives an epilogue.
 template <GemmEpi EPI>
-hipError_t launch_shape(const Nf4GemmArgs& a, hipStream_t stream) {
-    const auto tiles = [&](int64_t rows, int64_t tokens) {
-        return (a.n + rows - 1) / rows * ((a.m + tokens - 1) / tokens);
-    };
-    if constexpr (EPI == GemmEpi::kSwiGlu) {
-        // below half the chip in wide blocks (gate/up: up to 128 tokens) twice as many narrower ones
-        return tiles(128, 128) < 128 ? launch_tile<EPI, 2, 2, 2, 4>(a, 256, 1, stream)
-                                     : launch_tile<EPI, 4, 1, 2, 4>(a, 512, 1, stream);
+hipError_t launch_shape(const Nf4GemmArgs& a, const GemmPlan& plan, hipStream_t stream) {
+    constexpr bool kPairEpi = EPI == GemmEpi::kSwiGlu || EPI == GemmEpi::kQkvRope;
+    if (plan.shape == GemmShape::kWide) {
+        return launch_tile<EPI, 4, 1, 2, 4>(a, plan.splits, stream);
+    }
+    if constexpr (kPairEpi) {
+        if (plan.shape == GemmShape::kPair) {
+            return launch_tile<EPI, 2, 2, 2, 4>(a, plan.splits, stream);
+        }
     } else {
-        constexpr bool kRope = EPI == GemmEpi::kQkvRope;
-        if (tiles(128, 128) > 256) {
-            // a second, mostly empty round of 128 x 128 blocks costs more than fewer, larger blocks
-            return launch_tile<EPI, 4, 1, 2, 4>(a, 512, 1, stream);
-        }
-        // few tokens; or a short k in one unsplit round (no partial tiles, no reduce launch)
-        if (a.m <= 256 || (!kRope && a.k <= 4096 && tiles(128, 64) <= 256)) {
-            const hipError_t status = launch_tile<EPI, 4, 2, 1, 2>(a, 256, kRope ? 2 : 1, stream);
-            if (!kRope || status != hipErrorInvalidValue) {
-                return status;
-            }
-        }
-        if constexpr (kRope) {
-            // the rotation is in the reduce (two splits or more) or in blocks that hold pairs
-            if (tiles(128, 128) > 128) {
-                return launch_tile<EPI, 2, 2, 2, 4>(a, 256, 1, stream);
-            }
-            const hipError_t status = launch_tile<EPI, 4, 2, 1, 4>(a, 256, 2, stream);
-            return status != hipErrorInvalidValue ? status : launch_tile<EPI, 2, 2, 2, 4>(a, 256, 1, stream);
-        } else {
-            return launch_tile<EPI, 4, 2, 1, 4>(a, 256, 1, stream);
+        if (plan.shape == GemmShape::kLow) {
+            return launch_tile<EPI, 4, 2, 1, 2>(a, plan.splits, stream);
         }
     }
+    if constexpr (EPI != GemmEpi::kSwiGlu) {
+        if (plan.shape == GemmShape::kSquare) {
+            return launch_tile<EPI, 4, 2, 1, 4>(a, plan.splits, stream);
+        }
+    }
+    return hipErrorInvalidValue;
 }
-
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 }  // namespace
 
-// Everything the tile kernel reads or writes in 16-byte pieces is aligned to
-// them (rows are: n and k are multiples of 64 and 128), and a tile's lane
-// offsets and the grid fit 32 bits.  Other calls keep the 64-token kernels.
-bool nf4_tile_gemm_fits(GemmEpi epi, const Nf4GemmArgs& a) {
-    if (a.m < 1 || a.m > (int64_t{1} << 24) || a.n < 64 || a.n % 64 != 0 || a.n > (int64_t{1} << 24) || a.k < 128 ||
-        a.k % 128 != 0 || a.k > (int64_t{1} << 22) || a.m * a.n > (int64_t{1} << 40) || a.partials == nullptr) {
-        return false;
-    }
-    const bool rope = epi == GemmEpi::kQkvRope;
-    bool ok = aligned16(a.x) && aligned16(a.out) && aligned16(a.w[0]) && aligned16(a.partials);
-    if (epi == GemmEpi::kResidual || epi == GemmEpi::kResidualNorm) {
-        ok = ok && a.residual != nullptr && aligned16(a.residual);
-    }
-    if (epi == GemmEpi::kSwiGlu || rope) {
-        ok = ok && aligned16(a.w[1]);
-    }
-    if (rope) {
-        ok = ok && aligned16(a.w[2]) && aligned16(a.rope_cos) && aligned16(a.rope_sin) && aligned16(a.kcache) &&
-             aligned16(a.vcache) && a.q_rows % 128 == 0 && a.kv_rows % 128 == 0;
-    }
-    if (epi == GemmEpi::kResidualNorm) {
-        ok = ok && a.n == 2048;
-    }
-    return ok;
-}
-
-hipError_t launch_nf4_tile_gemm(GemmEpi epi, const Nf4GemmArgs& a, hipStream_t stream) {
+hipError_t launch_nf4_tile_gemm(GemmEpi epi, const Nf4GemmArgs& a, const GemmPlan& plan, hipStream_t stream) {
     switch (epi) {
         case GemmEpi::kBias:
-            return launch_shape<GemmEpi::kBias>(a, stream);
+            return launch_shape<GemmEpi::kBias>(a, plan, stream);
         case GemmEpi::kResidual:
-            return launch_shape<GemmEpi::kResidual>(a, stream);
+            return launch_shape<GemmEpi::kResidual>(a, plan, stream);
         case GemmEpi::kSwiGlu:
-            return launch_shape<GemmEpi::kSwiGlu>(a, stream);
+            return launch_shape<GemmEpi::kSwiGlu>(a, plan, stream);
         case GemmEpi::kQkvRope:
-            return launch_shape<GemmEpi::kQkvRope>(a, stream);
+            return launch_shape<GemmEpi::kQkvRope>(a, plan, stream);
         case GemmEpi::kResidualNorm:
-            return launch_shape<GemmEpi::kResidualNorm>(a, stream);
+            return launch_shape<GemmEpi::kResidualNorm>(a, plan, stream);
     }
     return hipErrorInvalidValue;
 }

@@ -1,4 +1,4 @@
-// NF4 GEMM on MFMA for few tokens (up to about 200): out[m, n] =
+// NF4 GEMM on MFMA for few tokens (gemm_few_plan() says how many): out[m, n] =
 // epilogue(sum_k x[m, k] * w[n, k]), w[n, k] = bf16(codebook[code] * absmax),
 // fp32 accumulation in v_mfma_f32_32x32x16_bf16.
 //
@@ -28,7 +28,7 @@
 //   down (k 11008)  11.8 -> 11.6 12.9 -> 12.3 16.4 -> 15.5 20.2 -> 18.6 21.6 -> 19.5
 //   gate alone      13.3 ->  9.1              22.8 -> 12.0
 #include "kc_device.h"
-#include "kc_kernels.h"
+#include "kc_gemm_plan.h"
 
 namespace kc {
 namespace {
@@ -459,7 +459,7 @@ __global__ __launch_bounds__(64 * (WN * WK + kLoaders)) void nf4_few_gemm_kernel
                 uint32_t ol[4], oh[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                                    if (bias != nullptr) {
+                    if (bias != nullptr) {
 #pragma unroll
                         for (int x = 0; x < 2; ++x) {
                             lo[2 * i + x] = lo[2 * i + x] + Bf16::load(bias[at + d + 2 * i + x]);
@@ -485,22 +485,12 @@ __global__ __launch_bounds__(64 * (WN * WK + kLoaders)) void nf4_few_gemm_kernel
     }
 }
 
-// Blocks that fill the chip: their LDS makes it one a CU.
-constexpr int64_t kBlocks = 256;
-
 template <GemmEpi EPI, int WN, int WK, int NT>
-hipError_t launch_few(const Nf4GemmArgs& a, int64_t splits, hipStream_t stream) {
-    constexpr int NF = EPI == GemmEpi::kSwiGlu ? 2 : 1;
-    const int64_t units = EPI == GemmEpi::kSwiGlu ? a.n / 16 : a.n / 32;
-    const int64_t m_tiles = (a.m + 32 * NT - 1) / (32 * NT);
-    const int64_t n_tiles = (units + WN - 1) / WN;
+hipError_t launch_few(const Nf4GemmArgs& a, int64_t S, hipStream_t stream) {
+    const int64_t fragments = EPI == GemmEpi::kSwiGlu ? a.n / 16 : a.n / 32;
+    const int64_t m_tiles = gemm_ceil(a.m, 32 * NT);
+    const int64_t n_tiles = gemm_ceil(fragments, WN);
     const int64_t steps = a.k / (kWindow * WK);
-    int64_t S = a.partials == nullptr ? 1 : splits;
-    S = S < steps ? S : steps;
-    while (S > 1 && NF * S * a.m * a.n > a.partial_floats) {
-        --S;
-    }
-    S = S > 1 ? S : 1;
     hipLaunchKernelGGL((nf4_few_gemm_kernel<EPI, WN, WK, NT>),
                        dim3(static_cast<unsigned>(n_tiles), static_cast<unsigned>(S), static_cast<unsigned>(m_tiles)),
                        dim3(64 * (WN * WK + kLoaders)), 0, stream, a, static_cast<int>(steps / S),
@@ -524,74 +514,49 @@ hipError_t launch_few(const Nf4GemmArgs& a, int64_t splits, hipStream_t stream) 
     return hipSuccess;
 }
 
-int64_t few_units(GemmEpi epi, const Nf4GemmArgs& a) { return epi == GemmEpi::kSwiGlu ? a.n / 16 : a.n / 32; }
-int64_t few_tiles(const Nf4GemmArgs& a) { return a.m <= 32 ? 1 : (a.m + 63) / 64; }
+template <GemmEpi EPI, int WN>
+hipError_t launch_few_tokens(const Nf4GemmArgs& a, const GemmPlan& plan, hipStream_t stream) {
+    return plan.tokens == 32 ? launch_few<EPI, WN, 4, 1>(a, plan.splits, stream)
+                             : launch_few<EPI, WN, 4, 2>(a, plan.splits, stream);
+}
 
-// A long k (down) is split over blocks of two fragments; its partial tiles cost
-// less than the k that a CU would walk alone.
-constexpr int64_t kLongK = 4096;
-
+// The shapes that gemm_few_plan() gives an epilogue (the 2048 and 2560 rows of the
+// row norm and of q, k and v never need three fragments a block).
 template <GemmEpi EPI>
-hipError_t launch_few_shape(const Nf4GemmArgs& a, hipStream_t stream) {
-    const int64_t units = few_units(EPI, a);
-    const int64_t tiles = few_tiles(a);
-    const bool one = a.m <= 32;
-    if (EPI == GemmEpi::kSwiGlu && a.m > 64 && (units + 1) / 2 * tiles > kBlocks) {
-        // gate/up of 65 .. 128 tokens: each weight formed once for all of them (two
-        // 64-token tiles of three fragments 31.5 us, this 22.3)
-        return launch_few<EPI, 3, 2, 4>(a, 1, stream);
+hipError_t launch_few_shape(const Nf4GemmArgs& a, const GemmPlan& plan, hipStream_t stream) {
+    if (plan.shape == GemmShape::kFew1) {
+        return launch_few_tokens<EPI, 1>(a, plan, stream);
     }
-    if (a.k > kLongK && EPI != GemmEpi::kSwiGlu) {
-        const int64_t splits = kBlocks / ((units + 1) / 2 * tiles);
-        return one ? launch_few<EPI, 2, 4, 1>(a, splits, stream) : launch_few<EPI, 2, 4, 2>(a, splits, stream);
+    if (plan.shape == GemmShape::kFew2) {
+        return launch_few_tokens<EPI, 2>(a, plan, stream);
     }
-    // a short k: as many fragments a block as make one round of blocks, unsplit (q of 64
-    // tokens 8.3 us in 64 blocks, 9.2 split in four); very few blocks (k, v) are split.
-    // A row norm needs a second launch either way, so o_proj splits over the whole
-    // chip and norms in its reduce (prefill of 9 layers, us, unsplit -> split: 1 token
-    // 505 -> 487, 16 511 -> 490, 48 629 -> 594, 64 643 -> 616)
-    if (units * tiles <= kBlocks) {
-        const int64_t fill = EPI == GemmEpi::kResidualNorm ? kBlocks : 64;
-        const int64_t splits = units * tiles < fill ? fill / (units * tiles) : 1;
-        return one ? launch_few<EPI, 1, 4, 1>(a, splits, stream) : launch_few<EPI, 1, 4, 2>(a, splits, stream);
+    if constexpr (EPI != GemmEpi::kResidualNorm && EPI != GemmEpi::kQkvRope) {
+        if (plan.shape == GemmShape::kFew3) {
+            return launch_few_tokens<EPI, 3>(a, plan, stream);
+        }
     }
-    if ((units + 1) / 2 * tiles <= kBlocks) {
-        return one ? launch_few<EPI, 2, 4, 1>(a, 1, stream) : launch_few<EPI, 2, 4, 2>(a, 1, stream);
+    if constexpr (EPI == GemmEpi::kSwiGlu) {
+        if (plan.shape == GemmShape::kFew3x128) {
+            return launch_few<EPI, 3, 2, 4>(a, plan.splits, stream);
+        }
     }
-    return one ? launch_few<EPI, 3, 4, 1>(a, 1, stream) : launch_few<EPI, 3, 4, 2>(a, 1, stream);
+    return hipErrorInvalidValue;
 }
 
 }  // namespace
 
-// Whole steps of four windows, and few enough tokens: one round of blocks (gate/up
-// of 160 tokens 40.8 us here, 38.9 in the tile kernel; a long k down to two splits).
-bool nf4_few_gemm_fits(GemmEpi epi, const Nf4GemmArgs& a) {
-    if (!nf4_tile_gemm_fits(epi, a) || a.k % 256 != 0) {
-        return false;
-    }
-    if (a.m <= 64) {
-        return true;
-    }
-    const int64_t units = few_units(epi, a);
-    const int64_t tiles = few_tiles(a);
-    if (epi == GemmEpi::kSwiGlu) {
-        return (units + 1) / 2 * tiles <= kBlocks || (a.m <= 128 && (units + 2) / 3 <= kBlocks);
-    }
-    return (units + 1) / 2 * tiles <= (a.k > kLongK ? kBlocks / 2 : kBlocks);
-}
-
-hipError_t launch_nf4_few_gemm(GemmEpi epi, const Nf4GemmArgs& a, hipStream_t stream) {
+hipError_t launch_nf4_few_gemm(GemmEpi epi, const Nf4GemmArgs& a, const GemmPlan& plan, hipStream_t stream) {
     switch (epi) {
         case GemmEpi::kBias:
-            return launch_few_shape<GemmEpi::kBias>(a, stream);
+            return launch_few_shape<GemmEpi::kBias>(a, plan, stream);
         case GemmEpi::kResidual:
-            return launch_few_shape<GemmEpi::kResidual>(a, stream);
+            return launch_few_shape<GemmEpi::kResidual>(a, plan, stream);
         case GemmEpi::kSwiGlu:
-            return launch_few_shape<GemmEpi::kSwiGlu>(a, stream);
+            return launch_few_shape<GemmEpi::kSwiGlu>(a, plan, stream);
         case GemmEpi::kQkvRope:
-            return launch_few_shape<GemmEpi::kQkvRope>(a, stream);
+            return launch_few_shape<GemmEpi::kQkvRope>(a, plan, stream);
         case GemmEpi::kResidualNorm:
-            return launch_few_shape<GemmEpi::kResidualNorm>(a, stream);
+            return launch_few_shape<GemmEpi::kResidualNorm>(a, plan, stream);
     }
     return hipErrorInvalidValue;
 }

@@ -181,13 +181,11 @@ hipError_t launch_nf4_gemm(GemmEpi epi, const Nf4GemmArgs& args, hipStream_t str
 // The second half of a split GEMM: a.partials [weights][splits][m][n] summed in
 // split order, then the epilogue.
 hipError_t launch_nf4_gemm_reduce(GemmEpi epi, const Nf4GemmArgs& args, int64_t splits, hipStream_t stream);
-// The same product for any token count (kc_gemm.hip), for calls that
-// nf4_tile_gemm_fits() accepts.
-bool nf4_tile_gemm_fits(GemmEpi epi, const Nf4GemmArgs& args);
-hipError_t launch_nf4_tile_gemm(GemmEpi epi, const Nf4GemmArgs& args, hipStream_t stream);
-// The same for few tokens (kc_gemm_few.hip), for calls that nf4_few_gemm_fits() accepts.
-bool nf4_few_gemm_fits(GemmEpi epi, const Nf4GemmArgs& args);
-hipError_t launch_nf4_few_gemm(GemmEpi epi, const Nf4GemmArgs& args, hipStream_t stream);
+// The same product for any token count (kc_gemm.hip) and for few tokens
+// (kc_gemm_few.hip), in the block shape and splits of gemm_plan() (kc_gemm_plan.h).
+struct GemmPlan;
+hipError_t launch_nf4_tile_gemm(GemmEpi epi, const Nf4GemmArgs& args, const GemmPlan& plan, hipStream_t stream);
+hipError_t launch_nf4_few_gemm(GemmEpi epi, const Nf4GemmArgs& args, const GemmPlan& plan, hipStream_t stream);
 
 // Row RMSNorm of m rows of 2048: out[r] = bf16((x[r] * inv_rms) * gamma), the
 // decode kernels' fp32 order.  With `embed`, row r is embed[tokens[start + r]]
@@ -221,7 +219,8 @@ struct PrefillAttnArgs {
     float* partials = nullptr;  // scratch of the matrix-core kernel's key splits
     int64_t partial_floats = 0;
 };
-// One block per query row and half of its heads: up to kAttnRowKeys cached rows.
+// One block per query row and half of its heads: up to kAttnRowKeys cached rows, and
+// any number of them for buffers that the matrix-core kernel cannot take.
 constexpr int64_t kAttnRowKeys = 128;
 hipError_t launch_prefill_attention(const PrefillAttnArgs& args, hipStream_t stream);
 // The same on the matrix cores (kc_prefill_attn.hip), for calls that

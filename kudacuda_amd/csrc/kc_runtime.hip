@@ -19,6 +19,7 @@
 
 #include "../../include/kudacuda.h"
 #include "kc_device.h"
+#include "kc_gemm_plan.h"
 #include "kc_kernels.h"
 
 namespace kc {
@@ -649,18 +650,14 @@ bool gemm_shape_ok(Handle* h, const char* symbol, int64_t tokens, int64_t in_fea
     return true;
 }
 
-// Few tokens (up to 64, more where they still make one round of its blocks) go
-// through kc_gemm_few.hip, more through the tile kernel, which forms each weight
-// once per 64 or 128 tokens in one launch.  Calls that neither can take (unaligned
-// buffers; k no multiple of 256 at up to 64 tokens) go in launches of
-// kGemmMaxTokens rows, whose waves keep a 16-row fragment for all of them.
+// The kernel that gemm_plan() picks; kParts is the one that goes in launches of
+// kGemmMaxTokens rows.
 hipError_t gemm_chunks(GemmEpi epi, Nf4GemmArgs a, int64_t tokens, hipStream_t stream) {
     a.m = tokens;
-    if (nf4_few_gemm_fits(epi, a)) {
-        return launch_nf4_few_gemm(epi, a, stream);
-    }
-    if (tokens > kGemmMaxTokens && nf4_tile_gemm_fits(epi, a)) {
-        return launch_nf4_tile_gemm(epi, a, stream);
+    const GemmPlan plan = gemm_plan(epi, a);
+    if (plan.shape != GemmShape::kParts) {
+        return plan.shape < GemmShape::kLow ? launch_nf4_few_gemm(epi, a, plan, stream)
+                                            : launch_nf4_tile_gemm(epi, a, plan, stream);
     }
     const uint16_t* x = a.x;
     const uint16_t* res = a.residual;

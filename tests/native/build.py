@@ -8,10 +8,11 @@
 * registry_smoke: a host program linked against kudacuda_amd/libkudacuda.so
   (rpath relative to this folder) that drives include/kudacuda_registry.h;
 * split_plan_check: a host program over the split-KV plan helpers of
-  kudacuda_amd/csrc/kc_kernels.h.
+  kudacuda_amd/csrc/kc_kernels.h;
+* libgemm_plan.so: the GEMM plan of kudacuda_amd/csrc/kc_gemm_plan.h.
 
-All are built here on the CPU and run by tests/test_registry.py and
-tests/test_split_plan.py.
+All are built here on the CPU and run by tests/test_registry.py,
+tests/test_split_plan.py and tests/test_gemm_plan.py.
 """
 
 from __future__ import annotations
@@ -30,6 +31,7 @@ PROBE = HERE / "registry_probe.hsaco"
 PROBE_COMPRESSED = HERE / "registry_probe_ccob.hsaco"
 SMOKE = HERE / "registry_smoke"
 SPLIT_PLAN = HERE / "split_plan_check"
+GEMM_PLAN = HERE / "libgemm_plan.so"
 
 
 def build() -> tuple[Path, ...]:
@@ -47,7 +49,9 @@ def build() -> tuple[Path, ...]:
     # host-only program over the split-plan helpers of kc_kernels.h
     subprocess.run([hipcc, "-O2", "-std=c++17", "-Wall", str(HERE / "split_plan_check.cpp"), "-o", str(SPLIT_PLAN)],
                    check=True, capture_output=True, text=True)
-    return PROBE, PROBE_COMPRESSED, SMOKE, SPLIT_PLAN
+    subprocess.run([hipcc, "-O2", "-std=c++17", "-Wall", "-fPIC", "-shared", str(HERE / "gemm_plan.cpp"), "-o",
+                    str(GEMM_PLAN)], check=True, capture_output=True, text=True)
+    return PROBE, PROBE_COMPRESSED, SMOKE, SPLIT_PLAN, GEMM_PLAN
 
 
 if __name__ == "__main__":
