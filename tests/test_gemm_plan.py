@@ -1,8 +1,9 @@
 """The GEMM dispatch (csrc/kc_gemm_plan.h) on the host.
 
-Over a wide grid every plan is one its launcher has: blocks within the chip
-where the rule says one round, partial tiles within the scratch, no empty split,
-pairs and rotations only in shapes that hold both fragments.
+The sizes of the GPU tests reach the block shapes and splits that they are there
+for, and over a wide grid every plan is one its launcher has: blocks within the
+chip where the rule says one round, partial tiles within the scratch, no empty
+split, pairs and rotations only in shapes that hold both fragments.
 """
 
 from __future__ import annotations
@@ -10,6 +11,8 @@ from __future__ import annotations
 import pytest
 
 from tests import _gemm_plan as P
+from tests import test_gpu_few_gemm as few
+from tests import test_gpu_tile_gemm as tile
 
 pytestmark = pytest.mark.skipif(not P.LIBRARY.exists(), reason="native checks not built (python tests/native/build.py)")
 SCRATCH_FLOATS = 4 << 20
@@ -21,6 +24,29 @@ POSSIBLE = {
     "swiglu": (*FEW, "pair", "wide"),
     "qkv_rope": ("few1", "few2", "square", "pair", "wide"),
 }
+
+
+def test_gpu_cases_reach_their_shapes():
+    for epilogue, cases in (("plain", tile.PLANS), ("residual", tile.PLANS), ("swiglu", tile.SWIGLU_PLANS),
+                            ("swiglu", tile.EXACT_PLANS), ("plain", few.PLANS), ("residual", few.PLANS),
+                            ("swiglu", few.SWIGLU_PLANS)):
+        for size, (shape, splits) in cases.items():
+            assert P.plan(epilogue, *size)[::2] == (shape, splits), (epilogue, size)
+    for count, (shape, splits) in tile.PREFILL_PLANS.items():
+        assert P.plan("qkv_rope", count, 2560, 2048)[::2] == (shape, splits), count
+
+
+def test_gpu_cases_reach_every_shape():
+    """... split and unsplit, with several windows a split, where a plan can be."""
+
+    def reached(cases):
+        return {(shape, splits > 1) for (_, _, k), (shape, splits) in cases.items()
+                if k // P.WINDOW[shape] > splits}
+
+    assert reached(tile.PLANS) >= {("low", False), ("low", True), ("square", False), ("square", True), ("wide", False)}
+    assert reached(tile.SWIGLU_PLANS) >= {("pair", False), ("pair", True), ("wide", False)}
+    assert reached(few.PLANS) >= {("few1", False), ("few1", True), ("few2", False), ("few2", True), ("few3", False)}
+    assert reached(few.SWIGLU_PLANS) >= {("few1", False), ("few1", True), ("few3", False), ("few3x128", False)}
 
 
 @pytest.mark.parametrize("epilogue", POSSIBLE)

@@ -2,7 +2,9 @@
 
 Sizes pick every block shape of its dispatch and the edges of each: one token, a
 token tile full or with one token, a last block with dead fragments, one step of
-K, fewer steps than prefetched, uneven splits.  The reference sums the same
+K, fewer steps than prefetched, uneven splits.  Beside each stands what the
+dispatch makes of it: (shape, splits of K), which tests/test_gemm_plan.py
+checks.  The reference sums the same
 bf16-rounded weights in fp64; the bound is one bf16 step of the output
 (tests/test_gpu_prefill.py::_close).
 """
@@ -20,18 +22,35 @@ pytestmark = pytest.mark.gpu
 SEED = 20260902
 
 
-@pytest.mark.parametrize("m,n,k", [
-    (1, 64, 256),        # one fragment a block, one step, one token
-    (32, 256, 2048),     # split over blocks of one fragment, a full token tile
-    (33, 2112, 1280),    # unsplit, one token in the second tile, five steps
-    (20, 9280, 256),     # two fragments a block
-    (64, 16448, 512),    # three fragments a block, one dead in the last block
-    (31, 16448, 768),    # the same, one token tile
-    (64, 2048, 11008),   # a long k: 43 steps over eight splits
-    (17, 64, 4352),      # a long k over 17 steps, one token tile
-    (193, 2048, 2304),   # four token tiles, one token in the last
-    (200, 192, 4608),    # a long k, four token tiles
-])
+PLANS = {
+    (1, 64, 256): ("few1", 1),       # one step, one token
+    (32, 256, 2048): ("few1", 8),    # a full token tile
+    (40, 192, 2816): ("few1", 10),   # eleven steps over ten splits
+    (33, 2112, 1280): ("few1", 1),   # one token in the second tile, five steps
+    (20, 9280, 256): ("few2", 1),
+    (64, 16448, 512): ("few3", 1),   # one fragment dead in the last block
+    (31, 16448, 768): ("few3", 1),   # the same, one token tile
+    (64, 2048, 11008): ("few2", 8),  # a long k: 43 steps over eight splits
+    (17, 64, 4352): ("few2", 17),    # a long k, one step a split, one token tile
+    (193, 2048, 2304): ("few1", 1),  # four token tiles, one token in the last
+    (200, 192, 4608): ("few2", 18),  # a long k, four token tiles
+    (512, 2048, 768): ("few2", 1),   # eight token tiles, three steps
+}
+SWIGLU_PLANS = {
+    (1, 64, 256): ("few1", 1),        # one step, one token
+    (1, 64, 1280): ("few1", 5),       # split: gate and up partials and their reduce
+    (40, 128, 2816): ("few1", 8),     # eleven steps over eight splits
+    (40, 1024, 512): ("few1", 1),
+    (64, 4160, 256): ("few2", 1),
+    (32, 8256, 768): ("few3", 1),     # one token tile
+    (63, 8256, 512): ("few3", 1),     # two token tiles
+    (65, 8256, 256): ("few3x128", 1),   # one token past 64
+    (128, 8192, 512): ("few3x128", 1),  # a full tile, two fragments alive in the last block
+    (256, 512, 256): ("few1", 1),     # four token tiles
+}
+
+
+@pytest.mark.parametrize("m,n,k", PLANS)
 @pytest.mark.parametrize("epi", ["plain", "bias", "residual"])
 def test_nf4_gemm_of_few_tokens_matches_fp64(torch_gpu, native, stream, m, n, k, epi):
     torch = torch_gpu
@@ -52,16 +71,7 @@ def test_nf4_gemm_of_few_tokens_matches_fp64(torch_gpu, native, stream, m, n, k,
     _close(host(out).reshape(m, n), want, inner=acc if epi == "residual" else None)
 
 
-@pytest.mark.parametrize("m,n,k", [
-    (1, 64, 256),       # one fragment a block, split
-    (40, 1024, 512),    # unsplit
-    (64, 4160, 256),    # two fragments a block
-    (32, 8256, 768),    # three, one token tile
-    (63, 8256, 512),    # three, two token tiles
-    (65, 8256, 256),    # 128-token tiles, one token past 64
-    (128, 8192, 512),   # a full one, two fragments alive in the last block
-    (256, 512, 256),    # four token tiles
-])
+@pytest.mark.parametrize("m,n,k", SWIGLU_PLANS)
 def test_nf4_gemm_swiglu_of_few_tokens_matches_fp64(torch_gpu, native, stream, m, n, k):
     torch = torch_gpu
     rng = np.random.default_rng([SEED, 7, m, n, k])

@@ -2,7 +2,8 @@
 
 Sizes pick every block shape of its dispatch and the edges of each: a last
 token tile with one token, a last row tile half empty, one K window, an odd
-number of windows, split and unsplit K.  The reference sums the same
+number of windows, split and unsplit K.  Beside each stands what the dispatch
+makes of it: (shape, splits of K), which tests/test_gemm_plan.py checks.  The reference sums the same
 bf16-rounded weights in fp64; the bound is one bf16 step of the output
 (tests/test_gpu_prefill.py::_close).
 """
@@ -20,15 +21,46 @@ pytestmark = pytest.mark.gpu
 SEED = 20260901
 
 
-@pytest.mark.parametrize("m,n,k", [
-    (65, 64, 128),       # low blocks: one window a K-group, half a row tile, one token in the last tile
-    (129, 192, 2048),    # low, split K
-    (300, 320, 384),     # low by the short k, three windows
-    (300, 192, 4224),    # square blocks, split K
-    (257, 2112, 4224),   # square, unsplit row tiles past half the chip
-    (705, 6208, 128),    # wide blocks: two windows, a quarter of the last row tile
-    (1025, 4160, 384),   # wide, one token in the last tile
-])
+PLANS = {
+    (65, 64, 128): ("low", 1),       # one window a K-group, half a row tile, one token in the last tile
+    (129, 192, 2048): ("few1", 3),   # (the few-token kernel)
+    (300, 320, 384): ("low", 3),     # one window a split
+    (300, 1088, 1152): ("low", 5),   # nine windows over five splits, half a row tile
+    (300, 3328, 1152): ("low", 1),   # nine windows
+    (100, 11008, 2048): ("low", 1),  # 16 windows
+    (300, 192, 4224): ("square", 33),
+    (257, 2112, 4224): ("square", 5),   # half a row tile
+    (300, 1152, 4224): ("square", 9),   # 33 windows over nine splits
+    (1100, 2048, 4224): ("square", 1),  # 33 windows, the residual stream's down projection
+    (705, 6208, 128): ("wide", 1),   # two windows, a quarter of the last row tile
+    (1025, 4160, 384): ("wide", 1),  # one token in the last tile
+}
+SWIGLU_PLANS = {
+    (65, 64, 256): ("few1", 1),      # (the few-token kernel)
+    (65, 64, 1152): ("pair", 9),     # one window a split
+    (127, 192, 128): ("pair", 1),    # one window a K-group
+    (200, 2048, 1152): ("pair", 3),  # nine windows over three splits
+    (300, 3840, 640): ("pair", 1),   # five windows
+    (1100, 1984, 128): ("wide", 1),  # half the last row tile
+    (1025, 1920, 384): ("wide", 1),  # six windows, one token in the last tile
+}
+EXACT_PLANS = {
+    (64, 8192, 256): ("few2", 1),
+    (500, 3968, 128): ("pair", 1),
+    (300, 11008, 128): ("wide", 1),
+}
+# one layer's q, k and v
+PREFILL_PLANS = {
+    200: ("few2", 1),
+    301: ("few2", 1),
+    385: ("square", 3),  # one token in the last tile
+    641: ("square", 2),
+    900: ("pair", 1),
+    1700: ("wide", 1),
+}
+
+
+@pytest.mark.parametrize("m,n,k", PLANS)
 @pytest.mark.parametrize("epi", ["plain", "bias", "residual"])
 def test_nf4_gemm_of_many_tokens_matches_fp64(torch_gpu, native, stream, m, n, k, epi):
     torch = torch_gpu
@@ -49,12 +81,7 @@ def test_nf4_gemm_of_many_tokens_matches_fp64(torch_gpu, native, stream, m, n, k
     _close(host(out).reshape(m, n), want, inner=acc if epi == "residual" else None)
 
 
-@pytest.mark.parametrize("m,n,k", [
-    (65, 64, 256),       # pair blocks, split K, half a row tile
-    (127, 192, 128),     # pair, one window a K-group
-    (1100, 1984, 128),   # wide blocks, half the last row tile
-    (1025, 1920, 384),   # wide, six windows, one token in the last tile
-])
+@pytest.mark.parametrize("m,n,k", SWIGLU_PLANS)
 def test_nf4_gemm_swiglu_of_many_tokens_matches_fp64(torch_gpu, native, stream, m, n, k):
     torch = torch_gpu
     rng = np.random.default_rng([SEED, 7, m, n, k])
@@ -70,11 +97,7 @@ def test_nf4_gemm_swiglu_of_many_tokens_matches_fp64(torch_gpu, native, stream, 
     _close(host(out).reshape(m, n), want)
 
 
-@pytest.mark.parametrize("m,n,k", [
-    (64, 8192, 256),     # the few-token kernel
-    (500, 3968, 128),    # pair blocks
-    (300, 11008, 128),   # wide blocks
-])
+@pytest.mark.parametrize("m,n,k", EXACT_PLANS)
 def test_swiglu_of_exact_sums_is_the_oracles(torch_gpu, native, stream, m, n, k):
     """Each token has two elements, powers of two 9 bits apart: the sums are exact,
     so every output is bf16(silu(gate) * up) of the oracle's fp32 silu to the bit,
@@ -106,11 +129,11 @@ def test_swiglu_of_exact_sums_is_the_oracles(torch_gpu, native, stream, m, n, k)
     assert np.array_equal(got, want)
 
 
-@pytest.mark.parametrize("count", [200, 301, 900, 1700])
+@pytest.mark.parametrize("count", PREFILL_PLANS)
 def test_prefill_rows_equal_those_of_64_token_parts(torch_gpu, native, count):
-    """One layer: a long prompt at once (q, k, v in low, square, pair and wide
-    blocks) writes the cache rows that its 64-token parts write, to the bound
-    of test_gpu_prefill (0.2 % of the elements more than one bf16 step apart)."""
+    """One layer: a long prompt at once (q, k, v in the blocks of PREFILL_PLANS)
+    writes the cache rows that its 64-token parts write, to the bound of
+    test_gpu_prefill (0.2 % of the elements more than one bf16 step apart)."""
 
     from kudacuda_amd import synthetic
     from kudacuda_amd.qwen2_decoder import Qwen2Nf4Decoder
