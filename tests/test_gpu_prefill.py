@@ -202,12 +202,13 @@ def test_model_prefill_matches_the_host_restatement(torch_gpu, prefill_pair):
 
 
 LONG_KW = dict(num_layers=2, vocab=4096, kv_capacity=128, token_capacity=128)
-LONG_PROMPT = 100  # two 64-token GEMM chunks (the second one ragged), causal rounds of 32 past 64
+LONG_PROMPT = 100  # two 64-token tiles of a GEMM block (the second one ragged), causal rounds of 32 past 64
 
 
 def test_model_prefill_of_a_multi_chunk_prompt(torch_gpu, native):
-    """A prompt longer than one GEMM launch: the second chunk's rows (and its
-    RoPE positions 64..99) and attention over 100 cached rows."""
+    """A prompt of more than one 64-token tile: the second tile's rows (and its
+    RoPE positions 64..99) and attention over 100 cached rows.  (Launches of 64
+    tokens one after the other: tests/test_gpu_gemm_parts.py.)"""
 
     from kudacuda_amd import synthetic
     from kudacuda_amd.qwen2_decoder import Qwen2Nf4Decoder
