@@ -99,6 +99,21 @@ __device__ __forceinline__ void unpack8(const uint4 v, float* out) {
     }
 }
 
+// Two fp32 values as bf16, the first in the low half (round to nearest even; NaN
+// stays NaN), by the hardware's conversion; and the halves of such a word in fp32.
+__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const bf16x2 v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
+    return __builtin_bit_cast(uint32_t, v);
+}
+__device__ __forceinline__ float lo_f32(uint32_t v) { return __uint_as_float(v << 16); }
+__device__ __forceinline__ float hi_f32(uint32_t v) { return __uint_as_float(v & 0xffff0000u); }
+
+// 32-bit word s of a uint4 (s known where the call is unrolled).
+__device__ __forceinline__ uint32_t word_of(const uint4& v, int s) {
+    return s == 0 ? v.x : (s == 1 ? v.y : (s == 2 ? v.z : v.w));
+}
+
 // ---------------------------------------------------------------------- exp2
 // 2^y by exact reduction y = n + f (n = rint(y), |f| <= 1/2, f exact) and the
 // degree-7 Taylor polynomial of e^(f ln 2) in Horner form, scaled by ldexp.

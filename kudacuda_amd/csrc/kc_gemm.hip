@@ -46,7 +46,6 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
-
 constexpr int kWindow = 64;     // k of one window and K-group: one absmax block
 
 template <int RF>
@@ -54,19 +53,6 @@ struct Codes {
     uint4 c[RF];
     float am[RF];
 };
-
-__device__ __forceinline__ uint32_t word_of(const uint4& v, int s) {
-    return s == 0 ? v.x : (s == 1 ? v.y : (s == 2 ? v.z : v.w));
-}
-
-// two fp32 values as bf16 (round to nearest even; NaN stays NaN)
-__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    const bf16x2 v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
-    return __builtin_bit_cast(uint32_t, v);
-}
-__device__ __forceinline__ float lo_f32(uint32_t v) { return __uint_as_float(v << 16); }
-__device__ __forceinline__ float hi_f32(uint32_t v) { return __uint_as_float(v & 0xffff0000u); }
 
 // A fragment's packed column pairs of one token (h[2 i4 + e]: columns 8 i4 +
 // 4 q + 2 e and the next) as 8 consecutive columns a lane: o[j] holds columns

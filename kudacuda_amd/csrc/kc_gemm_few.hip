@@ -45,18 +45,6 @@ struct Codes {
     float am;
 };
 
-__device__ __forceinline__ uint32_t word_of(const uint4& v, int s) {
-    return s == 0 ? v.x : (s == 1 ? v.y : (s == 2 ? v.z : v.w));
-}
-// two fp32 values as bf16 (round to nearest even; NaN stays NaN)
-__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    const bf16x2 v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
-    return __builtin_bit_cast(uint32_t, v);
-}
-__device__ __forceinline__ float lo_f32(uint32_t v) { return __uint_as_float(v << 16); }
-__device__ __forceinline__ float hi_f32(uint32_t v) { return __uint_as_float(v & 0xffff0000u); }
-
 // Row of its weight and the weight (seg) that row `fr` of fragment `unit` is.
 template <GemmEpi EPI>
 __device__ __forceinline__ int frag_row(const Nf4GemmArgs& a, int unit, int fr, int& seg) {

@@ -40,7 +40,6 @@ namespace kc {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int kHeads = 8;                 // query heads of a KV head
@@ -61,10 +60,6 @@ __device__ __forceinline__ float max_halves(float v) {
 __device__ __forceinline__ float sum_halves(float v) {
     const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(s[0]) + __uint_as_float(s[1]);
-}
-__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-    const bf16x2 v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
-    return __builtin_bit_cast(uint32_t, v);
 }
 
 // A block's results (columns: 8 tokens from row0 x 8 heads of KV head g) over
