@@ -157,9 +157,10 @@ KUDACUDA_API int kudacuda_nf4_gemv_bf16(void* handle, uint64_t input, uint64_t w
  * README.md:170).  output[m, n] = bf16(x[m] . Wbf16[n] + bias[n]) or, with
  * residual (then bias must be 0), bf16(residual[m, n] + bf16(x[m] . Wbf16[n]))
  * with Wbf16 = bf16(codebook[code] * absmax); fp32 accumulation.  residual may
- * alias output.  Contract: tokens>=1 (any count; processed 64 at a time),
- * out_features a positive multiple of 64, in_features a positive multiple of
- * 128, blocksize=64; x and output row-major [tokens, features] bf16. */
+ * alias output.  Contract: tokens>=1 (any count), out_features a positive
+ * multiple of 64, in_features a positive multiple of 128, blocksize=64; x and
+ * output row-major [tokens, features] bf16.  Buffers off a 16-byte boundary are
+ * accepted and run slower, in launches of 64 tokens. */
 KUDACUDA_API int kudacuda_nf4_gemm_bf16(void* handle, uint64_t input, uint64_t weight_packed, uint64_t absmax,
                                         uint64_t bias, uint64_t residual, uint64_t output, int64_t tokens,
                                         int64_t in_features, int64_t out_features, int64_t blocksize,

@@ -27,6 +27,7 @@
 //   q (k 2048)       7.3 ->  6.3  8.1 ->  6.6 10.1 ->  8.3 13.1 ->  8.3 14.2 ->  8.4
 //   down (k 11008)  11.8 -> 11.6 12.9 -> 12.3 16.4 -> 15.5 20.2 -> 18.6 21.6 -> 19.5
 //   gate alone      13.3 ->  9.1              22.8 -> 12.0
+// More tokens, against the tile kernel: the table at gemm_few_plan().
 #include "kc_device.h"
 #include "kc_gemm_plan.h"
 
