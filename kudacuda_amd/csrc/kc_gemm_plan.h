@@ -24,7 +24,7 @@ struct GemmPlan {
 };
 
 constexpr int64_t kGemmChip = 256;      // blocks that fill the chip, one a CU
-constexpr int64_t kGemmLongK = 4096;    // few tokens: a k from here on is split
+constexpr int64_t kGemmLongK = 4096;    // above it a k is long: see gemm_few_plan() and gemm_tile_plan()
 
 inline int64_t gemm_ceil(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
@@ -81,8 +81,7 @@ inline GemmPlan gemm_few_plan(GemmEpi epi, const Nf4GemmArgs& a) {
     const int64_t fragments = swiglu ? a.n / 16 : a.n / 32;
     const int64_t two = gemm_ceil(fragments, 2);
     const int64_t tiles = a.m <= 32 ? 1 : gemm_ceil(a.m, 64);
-    const bool long_k = a.k > kGemmLongK && !swiglu;
-    if (a.m > 64 && two * tiles > (long_k ? kGemmChip / 2 : kGemmChip)) {
+    if (a.m > 64 && two * tiles > (a.k > kGemmLongK && !swiglu ? kGemmChip / 2 : kGemmChip)) {
         // gate/up of 65 .. 128 tokens: each weight formed once for all of them (two
         // 64-token tiles of three fragments 31.5 us, this 22.3)
         if (swiglu && a.m <= 128 && gemm_ceil(fragments, 3) <= kGemmChip) {
@@ -90,20 +89,36 @@ inline GemmPlan gemm_few_plan(GemmEpi epi, const Nf4GemmArgs& a) {
         }
         return p;
     }
+    if (a.m <= 16 && fragments >= 2 * kGemmChip && a.k <= (fragments > 2 * kGemmChip ? 1024 : 768)) {
+        // all CUs full of two or three fragments and little k: the blocks' table and sums
+        // cost more than in kParts (gate/up of 1 token, 11008 rows: k 256 7.6 / 5.3 us, 512
+        // 8.7 / 6.6, 1024 10.6 / 9.1, 1536 even)
+        return p;
+    }
     p.tokens = a.m <= 32 ? 32 : 64;
     const int64_t steps = a.k / 256;
-    if (long_k) {
-        // a long k (down): its partial tiles cost less than the k that a CU would walk alone
+    const int64_t blocks = fragments * tiles;  // of one fragment
+    const bool few_blocks = blocks <= kGemmChip / 8;
+    if (a.k > kGemmLongK && !few_blocks && two * tiles <= kGemmChip) {
+        // a long k (down) over many blocks: two fragments a block and K over the chip (gate/up
+        // of 1024 rows, k 11008, 33 tokens: unsplit 29.8 us, 64-token launches 16.6, this 15)
         p.shape = GemmShape::kFew2;
         p.splits = gemm_splits(epi, a, kGemmChip / (two * tiles), steps);
-    } else if (fragments * tiles <= kGemmChip) {
-        // a short k: as many fragments a block as make one round of blocks, unsplit (q
-        // of 64 tokens 8.3 us in 64 blocks, 9.2 split in four); very few blocks (k, v)
-        // are split.  A row norm needs a second launch either way, so o_proj splits
-        // over the whole chip and norms in its reduce (prefill of 9 layers, us, unsplit
-        // -> split: 1 token 505 -> 487, 16 511 -> 490, 48 629 -> 594, 64 643 -> 616)
+    } else if (blocks <= kGemmChip) {
+        // A step of 256 costs 0.45 us (64 tokens 0.63), a split's partial tiles and reduce
+        // launch about 2: K is split past 2048 (2048 rows of 64 tokens, k 4096: 13.3 -> 10.5
+        // us, k 2048 8.3 -> 9.2) and, where few blocks leave most of the chip idle, from
+        // 1792 (1024 rows, k 2048: 6.9 in two splits, 6.1 in eight; k 1024 6.1 in two, 4.6
+        // unsplit).  Splits of one step only up to eight, sixteen at most: their planes cost
+        // the reduce (gate/up of 128 rows, k 4096: 8 splits 15 % faster than 16).  A row
+        // norm needs a second launch either way, so o_proj splits over the whole chip and
+        // norms in its reduce (prefill of 9 layers, us, unsplit -> split: 1 token 505 ->
+        // 487, 16 511 -> 490, 48 629 -> 594, 64 643 -> 616)
         p.shape = GemmShape::kFew1;
-        p.splits = gemm_splits(epi, a, (epi == GemmEpi::kResidualNorm ? kGemmChip : 64) / (fragments * tiles), steps);
+        if (epi == GemmEpi::kResidualNorm || a.k > 2048 || (a.k > 1536 && few_blocks)) {
+            const int64_t most = steps < 16 ? 8 : (steps < 32 ? steps / 2 : 16);
+            p.splits = gemm_splits(epi, a, kGemmChip / blocks < most ? kGemmChip / blocks : most, steps);
+        }
     } else {
         p.shape = two * tiles <= kGemmChip ? GemmShape::kFew2 : GemmShape::kFew3;
     }

@@ -46,12 +46,12 @@ def test_gpu_cases_reach_every_shape():
     assert reached(tile.PLANS) >= {("low", False), ("low", True), ("square", False), ("square", True), ("wide", False)}
     assert reached(tile.SWIGLU_PLANS) >= {("pair", False), ("pair", True), ("wide", False)}
     assert reached(few.PLANS) >= {("few1", False), ("few1", True), ("few2", False), ("few2", True), ("few3", False)}
-    assert reached(few.SWIGLU_PLANS) >= {("few1", False), ("few1", True), ("few3", False), ("few3x128", False)}
+    assert reached(few.SWIGLU_PLANS) >= {("few1", False), ("few1", True), ("few2", True), ("few3", False), ("few3x128", False)}
 
 
 @pytest.mark.parametrize("epilogue", POSSIBLE)
 def test_plans_are_ones_their_launchers_have(epilogue):
-    rows = {"qkv_rope": (2560,), "residual_norm": (2048,)}.get(epilogue, (64, 192, 1024, 2048, 8256, 11008, 22016))
+    rows = {"qkv_rope": (2560,), "residual_norm": (2048,)}.get(epilogue, (64, 192, 1024, 2048, 8256, 11008, 16384, 22016))
     depths = {"qkv_rope": (2048,), "residual_norm": (2048, 11008)}.get(epilogue, (128, 256, 384, 1152, 2048, 4352, 11008))
     counts = [*range(1, 140), *range(140, 1100, 31), 1999, 2049, 4096, 8192]
     for n in rows:
@@ -59,8 +59,9 @@ def test_plans_are_ones_their_launchers_have(epilogue):
             for m in counts:
                 shape, tokens, splits = P.plan(epilogue, m, n, k)
                 where = (m, n, k, shape, tokens, splits)
-                if shape == "parts":
-                    assert m <= 64 and k % 256 != 0, where
+                if shape == "parts":  # no whole steps, or all CUs full of two fragments and little k
+                    full = n // (16 if epilogue == "swiglu" else 32) >= 512
+                    assert m <= 64 and k % 256 != 0 or m <= 16 and k <= 1024 and full, where
                     continue
                 assert shape in POSSIBLE[epilogue], where
                 assert splits == 1 or (2 if epilogue == "swiglu" else 1) * splits * m * n <= SCRATCH_FLOATS, where

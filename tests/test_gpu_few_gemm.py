@@ -25,21 +25,24 @@ SEED = 20260902
 PLANS = {
     (1, 64, 256): ("few1", 1),       # one step, one token
     (32, 256, 2048): ("few1", 8),    # a full token tile
-    (40, 192, 2816): ("few1", 10),   # eleven steps over ten splits
+    (40, 192, 2816): ("few1", 8),    # eleven steps over eight splits
     (33, 2112, 1280): ("few1", 1),   # one token in the second tile, five steps
     (20, 9280, 256): ("few2", 1),
     (64, 16448, 512): ("few3", 1),   # one fragment dead in the last block
     (31, 16448, 768): ("few3", 1),   # the same, one token tile
     (64, 2048, 11008): ("few2", 8),  # a long k: 43 steps over eight splits
-    (17, 64, 4352): ("few2", 17),    # a long k, one step a split, one token tile
+    (17, 64, 4352): ("few1", 8),     # a long k over few blocks
+    (17, 2048, 4352): ("few2", 8),   # a long k, 17 steps, one token tile
     (193, 2048, 2304): ("few1", 1),  # four token tiles, one token in the last
-    (200, 192, 4608): ("few2", 18),  # a long k, four token tiles
+    (200, 192, 4608): ("few1", 9),   # a long k over few blocks, four token tiles
+    (100, 1088, 4352): ("few2", 7),  # a long k, two token tiles
     (512, 2048, 768): ("few2", 1),   # eight token tiles, three steps
 }
 SWIGLU_PLANS = {
     (1, 64, 256): ("few1", 1),        # one step, one token
-    (1, 64, 1280): ("few1", 5),       # split: gate and up partials and their reduce
+    (1, 64, 1792): ("few1", 7),       # split: gate and up partials and their reduce
     (40, 128, 2816): ("few1", 8),     # eleven steps over eight splits
+    (33, 1024, 4352): ("few2", 8),    # a long k: 17 steps over eight splits
     (40, 1024, 512): ("few1", 1),
     (64, 4160, 256): ("few2", 1),
     (32, 8256, 768): ("few3", 1),     # one token tile

@@ -1,6 +1,6 @@
 """GPU: the NF4 GEMM in launches of 64 tokens (csrc/kc_prefill.hip), which takes
-the calls whose buffers are not aligned to 16 bytes and, at up to 64 tokens, a k
-that is no multiple of 256; and the prefill over an unaligned workspace, which
+the calls whose buffers are not aligned to 16 bytes, at up to 64 tokens a k that
+is no multiple of 256, and at up to 16 tokens wide weights of little k; and the prefill over an unaligned workspace, which
 runs all of its GEMMs there and its attention row by row at any length.
 """
 
@@ -26,8 +26,9 @@ def _off(torch, bits, elements):
     return out
 
 
-# elements off alignment: 4 (8 bytes), which no other kernel takes; k = 128 at up to 64 tokens needs none
-@pytest.mark.parametrize("m,n,k,elements", [(100, 192, 2048, 4), (129, 64, 384, 4), (40, 320, 256, 4), (33, 192, 128, 0)])
+# elements off alignment: 4 (8 bytes), which no other kernel takes; the last two need none
+@pytest.mark.parametrize("m,n,k,elements", [(100, 192, 2048, 4), (129, 64, 384, 4), (40, 320, 256, 4), (33, 192, 128, 0),
+                                            (16, 16448, 512, 0)])
 @pytest.mark.parametrize("epi", ["plain", "bias", "residual", "swiglu"])
 def test_gemm_in_parts_matches_fp64(torch_gpu, native, stream, m, n, k, elements, epi):
     torch = torch_gpu

@@ -23,7 +23,7 @@ SEED = 20260901
 
 PLANS = {
     (65, 64, 128): ("low", 1),       # one window a K-group, half a row tile, one token in the last tile
-    (129, 192, 2048): ("few1", 3),   # (the few-token kernel)
+    (129, 192, 2048): ("few1", 8),   # (the few-token kernel)
     (300, 320, 384): ("low", 3),     # one window a split
     (300, 1088, 1152): ("low", 5),   # nine windows over five splits, half a row tile
     (300, 3328, 1152): ("low", 1),   # nine windows
