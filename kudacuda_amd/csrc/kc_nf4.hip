@@ -981,6 +981,14 @@ hipError_t launch_nf4_down11008(Act act, const Nf4DownArgs& a, hipStream_t strea
 
 namespace {
 bool aligned_to(const void* p, uintptr_t bytes) { return reinterpret_cast<uintptr_t>(p) % bytes == 0; }
+
+// Fewer elements leave the unit kernels too few waves: a thread's chain of 8 elements
+// and the block's table take longer than the element kernels' one element a thread.
+// us, element / unit kernel, of captured calls: quantise 131072 2.3 / 2.6, 262144 2.5 /
+// 2.7, 524288 3.1 / 2.7; to fp32 262144 2.2 / 2.3, 524288 2.5 / 2.5, 1048576 3.4 / 3.0;
+// to bf16 (its rounding by integer arithmetic) 524288 2.5 / 3.0, 1048576 3.2 / 3.1.
+constexpr int64_t kQuantizeUnits = int64_t{3} << 17;
+int64_t dequantize_units(int out_kind) { return int64_t{1} << (out_kind == 1 ? 20 : 19); }
 }  // namespace
 
 hipError_t launch_nf4_quantize_f32(const float* src, int64_t n, uint8_t* packed, float* absmax, hipStream_t stream) {
@@ -988,7 +996,7 @@ hipError_t launch_nf4_quantize_f32(const float* src, int64_t n, uint8_t* packed,
     if (nblocks <= 0) {
         return hipSuccess;
     }
-    if (aligned_to(src, 16) && aligned_to(packed, 4)) {
+    if (n >= kQuantizeUnits && aligned_to(src, 16) && aligned_to(packed, 4)) {
         hipLaunchKernelGGL(nf4_quantize8_kernel<float>, dim3(static_cast<unsigned>((8 * nblocks + 255) / 256)), dim3(256),
                            0, stream, src, 8 * nblocks, reinterpret_cast<uint32_t*>(packed), absmax);
         return hipGetLastError();
@@ -1004,7 +1012,7 @@ hipError_t launch_nf4_quantize_bf16(const uint16_t* src, int64_t n, uint8_t* pac
     if (nblocks <= 0) {
         return hipSuccess;
     }
-    if (aligned_to(src, 16) && aligned_to(packed, 4)) {
+    if (n >= kQuantizeUnits && aligned_to(src, 16) && aligned_to(packed, 4)) {
         hipLaunchKernelGGL(nf4_quantize8_kernel<uint16_t>, dim3(static_cast<unsigned>((8 * nblocks + 255) / 256)),
                            dim3(256), 0, stream, src, 8 * nblocks, reinterpret_cast<uint32_t*>(packed), absmax);
         return hipGetLastError();
@@ -1021,7 +1029,7 @@ hipError_t launch_nf4_dequantize(const uint8_t* packed, const float* absmax, int
     }
     // whole 8-element units within one absmax block, in aligned words (a block
     // size of 8 * 2^s: 64 in the NF4 format); anything else element by element
-    if (n % 8 == 0 && blocksize % 8 == 0 && (blocksize & (blocksize - 1)) == 0 && aligned_to(packed, 4) &&
+    if (n >= dequantize_units(out_kind) && n % 8 == 0 && blocksize % 8 == 0 && (blocksize & (blocksize - 1)) == 0 && aligned_to(packed, 4) &&
         aligned_to(out, 16)) {
         int shift = 0;
         while ((int64_t{8} << shift) < blocksize) {

@@ -1,6 +1,6 @@
 """GPU: NF4 quantise / dequantise by 8-element units against the oracle and,
-where the unit kernels do not apply (odd counts, unaligned buffers), against
-the element kernels.  Whole outputs, bit for bit."""
+where the unit kernels do not apply (small or odd counts, unaligned buffers),
+against the element kernels.  Whole outputs, bit for bit."""
 
 from __future__ import annotations
 
@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 SEED = 20260903
 
 
-@pytest.mark.parametrize("count", [64, 64 * 33, 64 * 257])
+# units from 393,216 elements on
+@pytest.mark.parametrize("count", [64, 64 * 33, 64 * 257, 393216 - 64, 393216, 393216 + 64 * 33])
 @pytest.mark.parametrize("dtype", [0, 1])
 def test_quantize_units_match_the_oracle_and_the_element_kernel(torch_gpu, native, stream, count, dtype):
     torch = torch_gpu
@@ -44,8 +45,16 @@ def test_quantize_units_match_the_oracle_and_the_element_kernel(torch_gpu, nativ
 
 
 @pytest.mark.parametrize("count,blocksize", [
-    (64, 64), (8, 8), (8192, 64), (8200, 64), (64 * 515, 64), (4096 + 8, 128), (2056, 1024),  # units
-    (8193, 64), (6, 64), (4096, 48),  # odd counts, a block size that is no power of two: element by element
+    # units of each kind (from 524,288 elements on, to bf16 from 1,048,576): whole blocks of threads, one
+    # unit past them, a ragged last block, other block sizes
+    (1 << 20, 64), ((1 << 20) + 8, 64), ((1 << 20) + 64 * 515, 64), ((1 << 20) + 8, 128), ((1 << 20) + 2056, 1024),
+    ((1 << 20) + 8, 8),
+    (1 << 19, 64), ((1 << 19) - 8, 64),  # to fp32 and fp16 the first of units, the last of elements
+    # odd counts, a block size that is no power of two: element by element
+    ((1 << 20) + 1, 64), ((1 << 20) + 48, 48),
+    # few elements: element by element
+    (64, 64), (8, 8), (8192, 64), (8200, 64), (64 * 515, 64), (4096 + 8, 128), (2056, 1024), (8193, 64), (6, 64),
+    (4096, 48),
 ])
 @pytest.mark.parametrize("kind", [0, 1, 2])
 def test_dequantize_units_and_elements_are_exact(torch_gpu, native, stream, count, blocksize, kind):
